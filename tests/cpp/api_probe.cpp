@@ -168,6 +168,34 @@ __attribute__((visibility("default"))) int probe_mha(int batch, int seq, int d_m
   return report(s, msg, msg_len);
 }
 
+// As probe_mha, with the window, prefix and softmax fields of the config.
+__attribute__((visibility("default"))) int probe_mha_masked(
+    int batch, int seq, int d_model, int heads, int kv_heads, int msl, int mask, int pos,
+    int window, int window_causal, int prefix_len, int softmax, int dtype, const float* Q,
+    const float* K, const float* V, const float* O, const float* x, float* attn, float* y,
+    char* msg, int msg_len) {
+  mha::Config cfg = mha::decoder_causal(d_model, heads, kv_heads);
+  cfg.max_seq_len = msl;
+  cfg.mask = mha::MaskKind(mask);
+  cfg.pos = mha::PosKind(pos);
+  cfg.causal = mask == 1;
+  cfg.window = window;
+  cfg.window_causal = window_causal != 0;
+  cfg.prefix_len = prefix_len;
+  cfg.softmax = mha::SoftmaxKind(softmax);
+  mha::Layer L;
+  Status s = mha::new_configured(cfg, DType(dtype), Q, K, V, O, &L);
+  if (!s) return report(s, msg, msg_len);
+  TensorF32 input, a, q;
+  input.shape = {batch, seq, d_model};
+  input.data.assign(x, x + (size_t)batch * seq * d_model);
+  s = mha::forward(L, input, &a, &q);
+  if (!s) return report(s, msg, msg_len);
+  copy_out(a, attn);
+  copy_out(q, y);
+  return report(s, msg, msg_len);
+}
+
 // dtype_name of an id into buf; dtype_implemented_forward as the result.
 __attribute__((visibility("default"))) int probe_dtype(int id, char* buf, int len) {
   const std::string_view n = dtype_name(DType(id));

@@ -31,6 +31,7 @@ def lib():
         L.probe_dense_backward.argtypes = [_i] * 6 + [_fp] * 5 + [_d, _fp, _cp, _i]
         L.probe_swiglu.argtypes = [_i] * 4 + [_fp] * 6 + [_cp, _i]
         L.probe_mha.argtypes = [_i] * 9 + [_fp] * 7 + [_cp, _i]
+        L.probe_mha_masked.argtypes = [_i] * 13 + [_fp] * 7 + [_cp, _i]
         L.probe_dtype.argtypes = [_i, _cp, _i]
         _LIB = L
     return _LIB
@@ -122,4 +123,13 @@ def mha(B, S, d, H, KVH, msl, mask, pos, dtype, Q, K, V, O, x):
     y = np.zeros((B * S, d), np.float32)
     check("probe_mha", B, S, d, H, KVH, msl, mask, pos, dtype, f(Q), f(K), f(V), f(O), f(x),
           f(attn), f(y))
+    return attn, y
+
+
+def mha_masked(B, S, d, H, KVH, msl, mask, pos, window, window_causal, prefix, softmax, dtype, Q,
+               K, V, O, x):
+    attn = np.zeros((B * S, d), np.float32)
+    y = np.zeros((B * S, d), np.float32)
+    check("probe_mha_masked", B, S, d, H, KVH, msl, mask, pos, window, window_causal, prefix,
+          softmax, dtype, f(Q), f(K), f(V), f(O), f(x), f(attn), f(y))
     return attn, y

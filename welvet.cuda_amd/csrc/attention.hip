@@ -7,11 +7,11 @@
 //   p == k_pos (mod msl): p = last - ((last - k_pos) mod msl);
 //   RoPE rotates Q and K at their global position (:487-504), ALiBi uses
 //   k_pos (:526-533); softmax or sigmoid over the allowed keys (:603-619).
-// The reference loop is serial f64 on one thread. Here the causal and
-// bidirectional masks without ALiBi run on the matrix cores (k_attn_mfma,
-// below); the other masks take k_attention, where one wave handles one
-// (token, head), keys are scored 64 at a time (one per lane), and the
-// softmax is accumulated online in fp32. RoPE is applied by the Q and K
+// The reference loop is serial f64 on one thread. Here head dims 32, 64 and
+// 128 run on the matrix cores (k_attn_mfma, below) for every mask; the other
+// head dims, and ALiBi under the sigmoid, take k_attention, where one wave
+// handles one (token, head), keys are scored 64 at a time (one per lane), and
+// the softmax is accumulated online in fp32. RoPE is applied by the Q and K
 // projections' GEMM epilogue when they run on the large tiles, else by
 // k_rope before either kernel.
 #include "common.h"
@@ -23,18 +23,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
-// x as three bf16 terms hi + mid + lo, each rounding the remainder of the
-// previous ones (to nearest even): x - hi - mid - lo is below 2^-24 |x|
-// (three 8-bit significands)
-__device__ __forceinline__ void split3(float x, __bf16 (&t)[3]) {
-  const __bf16 hi = (__bf16)x;
-  const float r1 = x - (float)hi;
-  const __bf16 mid = (__bf16)r1;
-  t[0] = hi;
-  t[1] = mid;
-  t[2] = (__bf16)(r1 - (float)mid);
-}
 
 __device__ __forceinline__ bool allow(int qp, int kp, const AttnArgs& a) {
   if (a.mask == 2) return true;
@@ -92,24 +80,19 @@ __global__ void k_rope(float* __restrict__ q, float* __restrict__ k, int tokens,
 
 constexpr int kMaxHdPerLane = 4;  // head_dim <= 256
 
-__global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
-  const int t = blockIdx.x;  // query token
-  const int h = blockIdx.y;  // query head
-  const int lane = threadIdx.x;
+// Attention of query token t, head h by one wave: keys scored 64 at a time
+// (one per lane) against their ring rows, online softmax in fp32. qs: the
+// query's hd values. Lane l ends with output dims l + 64 i in acc[i].
+__device__ __forceinline__ void attend_token(const AttnArgs& a, int t, int h, int lane,
+                                             const float* qs, float (&acc)[kMaxHdPerLane]) {
   const int b = t / a.seq;
   const int qp = t;
   const int kv_len = b * a.seq + a.seq;
   const int last = kv_len - 1;
   const int kvh = h / (a.heads / a.kv_heads);
-  const int qd = a.heads * a.hd, kvd = a.kv_heads * a.hd;
-  const float* qv = a.q + (size_t)t * qd + (size_t)h * a.hd;
-
-  __shared__ float qs[256];
-  for (int d = lane; d < a.hd; d += 64) qs[d] = qv[d];
-  __syncthreads();
+  const int kvd = a.kv_heads * a.hd;
 
   float m = -INFINITY, l = 0.0f;
-  float acc[kMaxHdPerLane];
 #pragma unroll
   for (int i = 0; i < kMaxHdPerLane; ++i) acc[i] = 0.0f;
   int n_allowed = 0;
@@ -172,18 +155,33 @@ __global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
       }
     }
   }
-  float* out = a.out + (size_t)t * qd + (size_t)h * a.hd;
   const float inv = (a.sigmoid || n_allowed == 0) ? 1.0f : 1.0f / l;
+#pragma unroll
+  for (int i = 0; i < kMaxHdPerLane; ++i) acc[i] = n_allowed == 0 ? 0.0f : acc[i] * inv;
+}
+
+__global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
+  const int t = blockIdx.x;  // query token
+  const int h = blockIdx.y;  // query head
+  const int lane = threadIdx.x;
+  const size_t row = (size_t)t * a.heads * a.hd + (size_t)h * a.hd;
+  __shared__ float qs[256];
+  for (int d = lane; d < a.hd; d += 64) qs[d] = a.q[row + d];
+  __syncthreads();
+  float acc[kMaxHdPerLane];
+  attend_token(a, t, h, lane, qs, acc);
+  float* out = a.out + row;
 #pragma unroll
   for (int i = 0; i < kMaxHdPerLane; ++i) {
     const int d = lane + 64 * i;
-    if (d < a.hd) out[d] = n_allowed == 0 ? 0.0f : acc[i] * inv;
+    if (d < a.hd) out[d] = acc[i];
   }
 }
 
 
 // ---------------------------------------------------------------------------
-// Matrix-core path for the causal and bidirectional masks without ALiBi.
+// Matrix-core path. The plain form (causal and bidirectional masks without
+// ALiBi) first; GEN, below, takes the other masks and ALiBi.
 //
 // Under the reference indexing a query of batch b scans key positions
 // kp in [0, b*seq + seq), and kp reads ring row p = last - ((last - kp) mod
@@ -197,10 +195,10 @@ __global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
 // Scores and sums are the same function of the same values; only the fp32
 // summation order differs from the per-position loop.
 //
-// A workgroup of 16 waves (8 at hd 128) takes 16 queries per wave of one
-// (batch, head) and walks the distinct rows in tiles of 64 keys staged in LDS in
-// matrix-core operand order, double-buffered through registers, one barrier
-// per tile. Per 16-key block a wave runs
+// A workgroup of 16, 8 or 4 waves (attn_waves_of) takes 16 queries per wave of
+// one (batch, head) and walks the distinct rows in tiles of 64 (or 32) keys staged
+// in LDS in matrix-core operand order, double-buffered through registers, one
+// barrier per tile. Per 16-key block a wave runs
 //   S^T = K Q^T  on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16, hd/32
 //                steps), Q and K each split into two bf16 terms hi + lo
 //                (x - hi - lo ~ 2^-17 |x|), and the three products down to
@@ -215,29 +213,130 @@ __global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
 // query, xor 16 / xor 32) and the rescaling of O happen once per 64 keys.
 // The softmax runs in base 2 (scores scaled by log2 e, weights from the
 // hardware exp2, within a few ulp of e^x).
-// Waves per workgroup, 16 queries each: 16 up to head_dim 64 (one
-// 1024-thread workgroup per CU, four waves per SIMD, each K/V tile staged
-// once for 256 queries: the B=8, S=512, 16x64 layer measured 0.1367 ms with
-// 8-wave workgroups, two per CU, and 0.1301 ms with 16), 8 for head_dim 128
-// (whose waves need more than 128 registers).
-constexpr int attn_waves(int hd) { return hd <= 64 ? 16 : 8; }
-constexpr int kKT = 64;  // keys per LDS tile
+//
+// GEN (ALiBi, the window and prefix masks, rings shorter than a tile): row p
+// stands for the positions p, p - msl, p - 2 msl, ... that lie in the
+// query's range [lo, hi] (every mask is such a range). With an ALiBi slope s
+// the positions at or below the query, kp0 - i msl for i < c, add
+//   e^(score - s (qp - kp0)) (1 + r + ... + r^(c - 1)),  r = e^(-s msl),
+// the same score with one factor, and a row above the query that may see it
+// (kp = p) adds its own term. Q, K, P and V take three bf16 terms there (six
+// products, down to 2^-24 relative): against 64 bits, with exact projections,
+// the output is 1e-7 off, as the fp32 loop of k_attention that it replaces.
+// That loop took one wave per (token, head) and one dependent V row per key:
+// 3 x 701 tokens, 12 heads of 64 over 4 K/V heads, causal with ALiBi: the layer
+// 1636 us, now 134 us (this kernel about 75 us; its matrix-core work is 20 us,
+// the softmax, the splits and the LDS traffic of two waves per SIMD the rest).
+// Keys per LDS tile: 64; 32 for GEN at 128 head dims (three terms of 64 keys
+// do not fit the LDS twice) and for the 4-wave workgroups whose 64 keys would
+// take more than half the LDS.
+constexpr int attn_keys(int hd, bool gen, int waves) {
+  return (hd > 64 && (gen || waves == 4)) || (gen && waves == 4) ? 32 : 64;
+}
 
-template <int HD, bool SIG>
-__global__ __launch_bounds__(64 * attn_waves(HD)) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 4 : 2, 8)))
+// Positions [lo, hi] that the mask allows to query qp (allow() as a range).
+__device__ __forceinline__ void key_range(const AttnArgs& a, int qp, int last, int& lo, int& hi) {
+  lo = 0;
+  hi = qp;
+  if (a.mask == 2) {
+    hi = last;
+  } else if (a.mask == 3) {
+    int w = a.window > 0 ? a.window : a.msl;
+    w = w < (1 << 30) ? w : 1 << 30;
+    lo = qp - w + 1 > 0 ? qp - w + 1 : 0;
+    if (!a.window_causal) hi = qp + w - 1 < last ? qp + w - 1 : last;
+  } else if (a.mask == 4 && qp < a.prefix_len) {
+    const int p1 = a.prefix_len - 1 < last ? a.prefix_len - 1 : last;
+    hi = p1 > qp ? p1 : qp;
+  }
+}
+
+// Positions of ring row p allowed to query qp: `count` of them at or below
+// the query, from `first` down in steps of msl (msl >= seq, so p - msl <= qp),
+// and `above` = 1 when p itself lies above the query and is allowed.
+__device__ __forceinline__ int key_count(const AttnArgs& a, int p, int qp, int last, int lo, int hi,
+                                         float inv_msl, int& first, int& above) {
+  above = 0;
+  first = p;
+  if (p > last) return 0;
+  if (p > qp) {
+    above = p <= hi ? 1 : 0;
+    first = p - a.msl;
+  }
+  const int n = first - lo;
+  if (n < 0) return 0;
+  int c = (int)((float)n * inv_msl);  // n / msl, at most one off
+  const int r = n - c * a.msl;
+  c += (r >= a.msl ? 1 : 0) - (r < 0 ? 1 : 0);
+  return c + 1;
+}
+
+// The ALiBi constants of a head: the slope in log2 units and, for the sums
+// over a row's positions, -log2(1 - r).
+struct Bias {
+  float sl2, x, lginv;
+};
+
+// log2(1 + r + ... + r^(c - 1)); log2(c) without ALiBi.
+__device__ __forceinline__ float log2_copies(int c, const Bias& s) {
+  if (s.sl2 == 0.0f) return __builtin_amdgcn_logf((float)c);
+  return __builtin_amdgcn_logf(1.0f - __builtin_amdgcn_exp2f(s.x * (float)c)) + s.lginv;
+}
+
+// log2 of the weight that row p's positions add to e^score for query qp;
+// -inf when none is allowed.
+__device__ __forceinline__ float log2_weight(const AttnArgs& a, int p, int qp, int last, int lo,
+                                             int hi, float inv_msl, const Bias& s) {
+  int first, above;
+  const int c = key_count(a, p, qp, last, lo, hi, inv_msl, first, above);
+  if (s.sl2 == 0.0f) return __builtin_amdgcn_logf((float)(c + above));  // log2(0) = -inf
+  const float below = c > 0 ? fmaf(-s.sl2, (float)(qp - first), log2_copies(c, s)) : -INFINITY;
+  if (!above) return below;
+  const float up = -s.sl2 * (float)(p - qp);
+  const float m = fmaxf(up, below);
+  return m + __builtin_amdgcn_logf(__builtin_amdgcn_exp2f(up - m) + __builtin_amdgcn_exp2f(below - m));
+}
+
+// x as T bf16 terms, each rounding the remainder of the ones before it (to
+// nearest even): two leave 2^-17 |x|, three 2^-25 |x|.
+template <int T>
+__device__ __forceinline__ void split_bf16(v4f x, bf16x4 (&t)[T]) {
+#pragma unroll
+  for (int k = 0; k < T; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      t[k][e] = (__bf16)x[e];
+      x[e] -= (float)t[k][e];
+    }
+}
+
+// acc + A B with both operands in T bf16 terms: the products a_i b_j with
+// i + j < T, the smallest first.
+template <int T>
+__device__ __forceinline__ v4f mfma_terms(const bf16x8 (&a)[T], const bf16x8 (&b)[T], v4f acc) {
+#pragma unroll
+  for (int s = T - 1; s >= 0; --s)
+#pragma unroll
+    for (int i = s; i >= 0; --i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[s - i], acc, 0, 0, 0);
+  return acc;
+}
+
+template <int HD, bool SIG, bool GEN, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? (GEN && HD > 64 ? 1 : 2) : WAVES / 4, 8)))
 void k_attn_mfma(AttnArgs a, int qblocks) {
+  constexpr int KT = attn_keys(HD, GEN, WAVES);         // keys per tile
+  constexpr int NB = KT / 16, NQ = KT / 32;             // 16-key blocks, 32-key groups
+  constexpr int TT = GEN ? 3 : 2;                       // bf16 terms of Q, K, V and P
   constexpr int KS = HD / 32;                           // QK MFMA steps (32 head dims)
   constexpr int DT = HD / 16;                           // 16-wide head-dim tiles of O
-  constexpr int kAttnWaves = attn_waves(HD);
-  constexpr int kQB = 16 * kAttnWaves;                  // queries per workgroup
-  constexpr int NT = 64 * kAttnWaves;                   // threads
-  // K in bf16 operand order: [16-key block kb][step ks][hi, lo][lane][8]:
+  constexpr int kQB = 16 * WAVES;                       // queries per workgroup
+  constexpr int NT = 64 * WAVES;                        // threads
+  // K in bf16 operand order: [16-key block kb][step ks][term][lane][8]:
   // lane 16 g + c16 holds key 16 kb + c16, head dims 32 ks + 8 g + j
-  constexpr int KBYTES = 4 * KS * 2 * 1024;
-  __shared__ __attribute__((aligned(16))) uint8_t ksb[2][KBYTES];
-  // V in bf16 operand order: [32-key group q][head-dim tile dt][hi, lo][lane][8]
-  constexpr int VBYTES = 2 * DT * 2 * 1024;
-  __shared__ __attribute__((aligned(16))) uint8_t vsb[2][VBYTES];
+  constexpr int KBYTES = NB * KS * TT * 1024;
+  // V in bf16 operand order: [32-key group q][head-dim tile dt][term][lane][8]
+  constexpr int VBYTES = NQ * DT * TT * 1024;
+  __shared__ __attribute__((aligned(16))) uint8_t ksb[2][KBYTES], vsb[2][VBYTES];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c16 = lane & 15, g = lane >> 4;
   const int b = blockIdx.x / qblocks, qb = blockIdx.x % qblocks;
@@ -254,10 +353,24 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
   // the sigmoid variant works in natural units
   const float scale_log2 = (float)(a.scale * 1.4426950408889634);
   const float scale_nat = (float)a.scale;
+  // GEN: key positions [lo, hi] allowed to this lane's query, and the ALiBi
+  // slope in log2 units
+  int lo = 0, hi = 0;
+  float inv_msl = 0.0f;
+  Bias al = {0.0f, 0.0f, 0.0f};
+  if constexpr (GEN) {
+    key_range(a, qp, last, lo, hi);
+    inv_msl = 1.0f / (float)a.msl;
+    if (a.alibi) {
+      al.sl2 = (float)(exp2(-(double)(h + 1) * 8.0 / (double)a.heads) * 1.4426950408889634);
+      al.x = -al.sl2 * (float)a.msl;
+      al.lginv = -__builtin_amdgcn_logf(1.0f - __builtin_amdgcn_exp2f(al.x));
+    }
+  }
 
   // Q operand: lane (query c16, group g), head dims 32 ks + 8 g + j, as
-  // two bf16 terms (hi and the rounded remainder: 16 significand bits, as K)
-  bf16x8 qop[KS][2];
+  // TT bf16 terms (each the rounded remainder of those before it)
+  bf16x8 qop[KS][TT];
   {
     const float* qrow = a.q + (size_t)qp * qd + (size_t)h * HD;
 #pragma unroll
@@ -265,10 +378,13 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       const v4f q0 = *reinterpret_cast<const v4f*>(qrow + 32 * ks + 8 * g);
       const v4f q1 = *reinterpret_cast<const v4f*>(qrow + 32 * ks + 8 * g + 4);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        __bf16 t3[3];
-        split3(j < 4 ? q0[j] : q1[j - 4], t3);
-        qop[ks][0][j] = t3[0], qop[ks][1][j] = t3[1];
+      for (int half = 0; half < 2; ++half) {
+        bf16x4 t[TT];
+        split_bf16<TT>(half ? q1 : q0, t);
+#pragma unroll
+        for (int k = 0; k < TT; ++k)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) qop[ks][k][4 * half + j] = t[k][j];
       }
     }
   }
@@ -277,12 +393,12 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
   for (int d = 0; d < DT; ++d) o[d] = v4f{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.0f;
 
-  // K and V rows of a tile in pair units: unit i = tid + NT u covers row
+  // K rows of a tile in pair units: unit i = tid + NT u covers row
   // i / (HD/8) and the column quads c4 and c4 + HD/2, c4 = 4 (i % (HD/8)).
   // Rows past `last` are exact zeros (a tile wholly past it is a zero tile:
   // the loads stay unconditional).
-  constexpr int UNITS = kKT * HD / 8, PU = (UNITS + NT - 1) / NT;
-  v4f kreg[2 * PU], vreg[2 * PU];
+  constexpr int UNITS = KT * HD / 8, PU = (UNITS + NT - 1) / NT;
+  v4f kreg[2 * PU];
   auto load_k = [&](int t0) {
 #pragma unroll
     for (int u = 0; u < PU; ++u) {
@@ -298,25 +414,29 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       kreg[2 * u + 1] = p <= last ? k1 : z;
     }
   };
+  // V of a tile in units of 4 rows x 1 column: unit i = tid + NT u covers
+  // rows 4 (i / HD) .. + 3 of column i % HD (every load instruction of a wave
+  // reads whole rows), so that the 4 values, neighbours in the operand
+  // order, are stored with one 8-byte write per term.
+  constexpr int VUNITS = KT / 4 * HD, PV = (VUNITS + NT - 1) / NT;
+  v4f vreg[PV];
   auto load_v = [&](int t0) {
 #pragma unroll
-    for (int u = 0; u < PU; ++u) {
+    for (int u = 0; u < PV; ++u) {
       const int i = tid + NT * u;
-      if (UNITS % NT != 0 && i >= UNITS) break;
-      const int r = i / (HD / 8), c4 = (i % (HD / 8)) * 4;
-      const int p = t0 + r, pc = p <= last ? p : last;
-      const size_t off = (size_t)pc * kvd + (size_t)kvh * HD + c4;
-      const v4f v0 = *reinterpret_cast<const v4f*>(a.v + off);
-      const v4f v1 = *reinterpret_cast<const v4f*>(a.v + off + HD / 2);
-      const v4f z = v4f{0.f, 0.f, 0.f, 0.f};
-      vreg[2 * u] = p <= last ? v0 : z;
-      vreg[2 * u + 1] = p <= last ? v1 : z;
+      if (VUNITS % NT != 0 && i >= VUNITS) break;  // whole waves
+      const float* src = a.v + (size_t)kvh * HD + i % HD;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int p = t0 + 4 * (i / HD) + e, pc = p <= last ? p : last;
+        const float v = src[(size_t)pc * kvd];
+        vreg[u][e] = p <= last ? v : 0.0f;
+      }
     }
   };
   // K row r, head dims d..d+3 (d = c4 or c4 + HD/2, a multiple of 4) go to
   // block r / 16, step d / 32, lane 16 ((d / 8) % 4) + r % 16, elements
-  // d % 8 .. + 3: one 8-byte store per term. K takes two bf16 terms, hi and
-  // lo = bf16(k - hi) (k - hi is exact): k to ~2^-17 relative.
+  // d % 8 .. + 3: one 8-byte store per term.
   auto store_k = [&](int buf) {
 #pragma unroll
     for (int u = 0; u < PU; ++u) {
@@ -326,21 +446,12 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const int d = c4 + half * (HD / 2);
-        __bf16 t[2][4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float k = kreg[2 * u + half][e];
-          const __bf16 hi = (__bf16)k;
-          t[0][e] = hi;
-          t[1][e] = (__bf16)(k - (float)hi);
-        }
-        uint8_t* dst = ksb[buf] + (size_t)(((r >> 4) * KS + (d >> 5)) * 2) * 1024 +
+        bf16x4 t[TT];
+        split_bf16<TT>(kreg[2 * u + half], t);
+        uint8_t* dst = ksb[buf] + (size_t)(((r >> 4) * KS + (d >> 5)) * TT) * 1024 +
                        (((d >> 3) & 3) * 16 + (r & 15)) * 16 + (d & 7) * 2;
 #pragma unroll
-        for (int term = 0; term < 2; ++term) {
-          bf16x4 v = {t[term][0], t[term][1], t[term][2], t[term][3]};
-          *reinterpret_cast<bf16x4*>(dst + term * 1024) = v;
-        }
+        for (int term = 0; term < TT; ++term) *reinterpret_cast<bf16x4*>(dst + term * 1024) = t[term];
       }
     }
   };
@@ -348,42 +459,36 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
   // products: 32-key group q = r / 32, and within it the lane group g and
   // element j that also hold that key's weight in the score layout (key
   // 16 kb + 4 g + i of the group <-> g, j = 4 kb + i); lane 16 g + d % 16 of
-  // head-dim tile d / 16. Each value is stored as bf16 hi and lo = v - hi.
+  // head-dim tile d / 16.
   auto store_v = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < PU; ++u) {
+    for (int u = 0; u < PV; ++u) {
       const int i = tid + NT * u;
-      if (UNITS % NT != 0 && i >= UNITS) break;
-      const int r = i / (HD / 8), c4 = (i % (HD / 8)) * 4;
-      const int q = r >> 5, rr = r & 31;
-      const int gk = (rr >> 2) & 3, j = 4 * (rr >> 4) + (rr & 3);
+      if (VUNITS % NT != 0 && i >= VUNITS) break;
+      const int d = i % HD, r4 = i / HD;  // rows 4 r4 ..: group q, j = 4 (rr / 16) + 0..3
+      const int q = r4 >> 3, rr4 = r4 & 7;
+      bf16x4 t[TT];
+      split_bf16<TT>(vreg[u], t);
+      uint8_t* dst = vsb[buf] + (size_t)((q * DT + (d >> 4)) * TT) * 1024 +
+                     ((rr4 & 3) * 16 + (d & 15)) * 16 + (rr4 >> 2) * 8;
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int d = c4 + e + half * (HD / 2);
-          const float v = vreg[2 * u + half][e];
-          const __bf16 hi = (__bf16)v, lo = (__bf16)(v - (float)hi);
-          uint8_t* dst = vsb[buf] + (size_t)((q * DT + (d >> 4)) * 2) * 1024 + (gk * 16 + (d & 15)) * 16 + j * 2;
-          *reinterpret_cast<__bf16*>(dst) = hi;
-          *reinterpret_cast<__bf16*>(dst + 1024) = lo;
-        }
+      for (int term = 0; term < TT; ++term) *reinterpret_cast<bf16x4*>(dst + term * 1024) = t[term];
     }
   };
-  // S^T of a tile: 4 blocks of 16 keys; K (hi, lo) times Q (hi, lo): the
-  // three products down to 2^-16 relative, the small ones first
-  auto scores = [&](const uint8_t* kt, v4f (&sc)[4]) {
+  // S^T of a tile: blocks of 16 keys; K terms times Q terms, the small
+  // products first: with two terms each the three down to 2^-16 relative, with
+  // three the six down to 2^-24
+  auto scores = [&](const uint8_t* kt, v4f (&sc)[NB]) {
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < NB; ++kb) {
       sc[kb] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const uint8_t* kp = kt + (size_t)((kb * KS + ks) * 2) * 1024 + lane * 16;
-        const bf16x8 kh = *reinterpret_cast<const bf16x8*>(kp);
-        const bf16x8 kl = *reinterpret_cast<const bf16x8*>(kp + 1024);
-        sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qop[ks][0], sc[kb], 0, 0, 0);
-        sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qop[ks][1], sc[kb], 0, 0, 0);
-        sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qop[ks][0], sc[kb], 0, 0, 0);
+        const uint8_t* kp = kt + (size_t)((kb * KS + ks) * TT) * 1024 + lane * 16;
+        bf16x8 k[TT];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) k[t] = *reinterpret_cast<const bf16x8*>(kp + t * 1024);
+        sc[kb] = mfma_terms<TT>(k, qop[ks], sc[kb]);
       }
     }
   };
@@ -399,18 +504,23 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
   // was last read before the previous barrier). All loads are unconditional
   // (a tile past the range is a zero tile, stored but never read).
 #pragma unroll 1
-  for (int t0 = p_lo, cur = 0; t0 <= last; t0 += kKT, cur ^= 1) {
-    load_k(t0 + kKT);
-    load_v(t0 + kKT);
+  for (int t0 = p_lo, cur = 0; t0 <= last; t0 += KT, cur ^= 1) {
+    load_k(t0 + KT);
+    load_v(t0 + KT);
     const uint8_t* vt = vsb[cur];
-    // multiplicity base of the tile start: floor(t0 / msl) + 1 (msl >= 64, so
-    // the tile crosses at most one multiple of msl)
+    // multiplicity base of the tile start: floor(t0 / msl) + 1 (msl >= KT
+    // without GEN, so the tile crosses at most one multiple of msl)
     const int base0 = t0 / a.msl + 1;
     const int next_mult = base0 * a.msl;  // first p with a larger base
     // multiplicity of the row of key k (block kb, lane key i) for this query
     const float base0f = (float)base0;
     auto mult = [&](int kb, int i) {
       const int p = t0 + 16 * kb + 4 * g + i;
+      if constexpr (GEN) {
+        int first, above;
+        const int c = key_count(a, p, qp, last, lo, hi, inv_msl, first, above);
+        return (float)(c + above);
+      }
       const float c = p <= last ? base0f + (p >= next_mult ? 1.0f : 0.0f) : 0.0f;
       return c - (causal && p > qp ? 1.0f : 0.0f);
     };
@@ -418,21 +528,35 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
     // inside [p_lo, last], not crossing a multiple of msl, and wholly at or
     // below (c = base) or wholly above (c = base - 1, causal) the wave's 16
     // queries. cu is that value (wave-uniform), or -1 for per-key values; a
-    // tile with cu == 0 adds nothing to this wave's queries.
-    const int kmax = t0 + kKT - 1;
+    // tile with cu == 0 adds nothing to this wave's queries. GEN: the same
+    // from the first and the last query's ranges (both grow with the query);
+    // first0 is the first position that the tile's first row stands for.
+    const int kmax = t0 + KT - 1;
     const int qw0 = b * a.seq + qb * kQB + __builtin_amdgcn_readfirstlane(wave) * 16;
-    int cu = -1;
-    if (kmax <= last && next_mult > kmax) {
+    int cu = -1, first0 = t0;
+    if constexpr (GEN) {
+      const int qw1 = qw0 + 15 < last ? qw0 + 15 : last;  // the wave's last query
+      int l0, h0, l1, h1;
+      key_range(a, qw0 < last ? qw0 : last, last, l0, h0);
+      key_range(a, qw1, last, l1, h1);
+      const bool above = t0 > qw1 && t0 > h1;
+      if (kmax <= last && (kmax <= qw0 || above)) {
+        first0 = above ? t0 - a.msl : t0;
+        const int n0 = first0 - l1, n1 = first0 + KT - 1 - l0;  // least and largest
+        if (n1 < 0) cu = 0;
+        else if (n0 >= 0 && n0 / a.msl == n1 / a.msl) cu = n0 / a.msl + 1;
+      }
+    } else if (kmax <= last && next_mult > kmax) {
       if (!causal || kmax <= qw0) cu = base0;
       else if (t0 > qw0 + 15) cu = base0 - 1;
     }
     if (cu != 0) {  // wave-uniform
-    v4f sc[4];
+    v4f sc[NB];
     scores(ksb[cur], sc);
-    float w[16];
+    float w[4 * NB];
     if constexpr (SIG) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float c = cu > 0 ? (float)cu : mult(kb, i);
@@ -442,10 +566,32 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       // base-2 scores with the multiplicity folded into the exponent
       // (c 2^x = 2^(x + log2 c)); masked keys at -inf
       float smax = -INFINITY;
-      if (cu > 0) {
+      if (GEN && cu > 0) {
+        // ALiBi: the distance to the row's first position, then the sum over
+        // its cu positions as one factor (log2_copies)
+        const float lc = log2_copies(cu, al);
+        const float d0 = (float)(qp - first0 - 4 * g);
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float bias = fmaf(-al.sl2, d0 - (float)(16 * kb + i), lc);
+            w[4 * kb + i] = fmaf(sc[kb][i], scale_log2, bias);
+            smax = fmaxf(smax, w[4 * kb + i]);
+          }
+      } else if (GEN) {
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float bias = log2_weight(a, t0 + 16 * kb + 4 * g + i, qp, last, lo, hi, inv_msl, al);
+            w[4 * kb + i] = bias > -INFINITY ? fmaf(sc[kb][i], scale_log2, bias) : -INFINITY;
+            smax = fmaxf(smax, w[4 * kb + i]);
+          }
+      } else if (cu > 0) {
         const float lc = __builtin_amdgcn_logf((float)cu);
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             w[4 * kb + i] = sc[kb][i] * scale_log2 + lc;
@@ -453,7 +599,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
           }
       } else {
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const float c = mult(kb, i);
@@ -468,7 +614,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       const float corr = __builtin_amdgcn_exp2f(m - nz);  // m = -inf: 0
       float ws = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
+      for (int i = 0; i < 4 * NB; ++i) {
         w[i] = __builtin_amdgcn_exp2f(w[i] - nz);
         ws += w[i];
       }
@@ -480,28 +626,30 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       m = nm;
     }
     // O^T += V^T P^T on the bf16 matrix cores, 32 keys per product, each
-    // operand split into bf16 hi + lo: hi*hi + hi*lo + lo*hi (the dropped
-    // lo*lo term and the split leave ~2^-16 relative error per product).
+    // operand split into TT bf16 terms as the scores' operands (with two, the
+    // dropped lo*lo product and the split leave ~2^-16 relative error).
     // Lane (query c16, group g) passes the weights it already holds: element
     // j of group g is key 16 (2q + j / 4) + 4g + j % 4 of the tile.
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      bf16x8 ph, pl;
+    for (int q = 0; q < NQ; ++q) {
+      bf16x8 p[TT];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float wv = w[4 * (2 * q + (j >> 2)) + (j & 3)];
-        const __bf16 h = (__bf16)wv;
-        ph[j] = h;
-        pl[j] = (__bf16)(wv - (float)h);
+      for (int j2 = 0; j2 < 2; ++j2) {
+        const float* wq = w + 4 * (2 * q + j2);
+        bf16x4 t[TT];
+        split_bf16<TT>(v4f{wq[0], wq[1], wq[2], wq[3]}, t);
+#pragma unroll
+        for (int term = 0; term < TT; ++term)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) p[term][4 * j2 + j] = t[term][j];
       }
 #pragma unroll
       for (int d = 0; d < DT; ++d) {
-        const uint8_t* vb = vt + (size_t)((q * DT + d) * 2) * 1024 + lane * 16;
-        const bf16x8 vh = *reinterpret_cast<const bf16x8*>(vb);
-        const bf16x8 vl = *reinterpret_cast<const bf16x8*>(vb + 1024);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, ph, o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, pl, o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vl, ph, o[d], 0, 0, 0);
+        const uint8_t* vb = vt + (size_t)((q * DT + d) * TT) * 1024 + lane * 16;
+        bf16x8 v[TT];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) v[t] = *reinterpret_cast<const bf16x8*>(vb + t * 1024);
+        o[d] = mfma_terms<TT>(v, p, o[d]);
       }
     }
     }
@@ -509,21 +657,57 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
     store_v(cur ^ 1);
     __syncthreads();
   }
-  if (!q_ok) return;
   // o[d]: lane holds query c16, head dims d*16 + 4g + i
   const float inv = SIG ? 1.0f : (l > 0.0f ? 1.0f / l : 0.0f);
-  float* out = a.out + (size_t)qp * qd + (size_t)h * HD;
   // with a.split (seq % 16 == 0: the wave's 16 queries are rows 16 rb ..
   // 16 rb + 15, all valid), the outputs are also staged in LDS, which the
   // K/V tiles no longer use after the loop's last barrier: 64 HD bytes per
-  // wave, waves 0-7 in ksb and 8-15 in vsb
-  float* stg = reinterpret_cast<float*>(wave < 8 ? &ksb[0][0] + wave * 64 * HD
-                                                 : &vsb[0][0] + (wave - 8) * 64 * HD);
+  // wave, the first half of the waves in ksb and the others in vsb
+  constexpr int HW = WAVES / 2;
+  static_assert(HW * 64 * HD <= 2 * KBYTES && HW * 64 * HD <= 2 * VBYTES, "output staging");
+  float* stg = reinterpret_cast<float*>(wave < HW ? &ksb[0][0] + wave * 64 * HD
+                                                  : &vsb[0][0] + (wave - HW) * 64 * HD);
+  bool redo = false;
+  if constexpr (GEN) {
+    // A key or value that is not finite (or near the f32 maximum, where a
+    // bf16 term overflows) puts NaN into the products of every query of the
+    // tile, also of those that may not see it: such a wave takes its queries
+    // again, one by one over the allowed keys only.
+    float t = SIG ? 0.0f : l - l;
+    if (!SIG && !(l > 0.0f)) t = NAN;
 #pragma unroll
-  for (int d = 0; d < DT; ++d) {
-    const float4 v = make_float4(o[d][0] * inv, o[d][1] * inv, o[d][2] * inv, o[d][3] * inv);
-    *reinterpret_cast<float4*>(out + d * 16 + 4 * g) = v;
-    if (a.split) *reinterpret_cast<float4*>(stg + c16 * HD + d * 16 + 4 * g) = v;
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t += o[d][i] - o[d][i];
+    redo = __any(q_ok && t != 0.0f);
+  }
+  if (redo) {
+    for (int j = 0; j < 16; ++j) {
+      const int sj = qb * kQB + wave * 16 + j;
+      if (sj >= a.seq) break;  // wave-uniform
+      const int t = b * a.seq + sj;
+      const size_t row = (size_t)t * qd + (size_t)h * HD;
+      float acc[kMaxHdPerLane];
+      attend_token(a, t, h, lane, a.q + row, acc);
+#pragma unroll
+      for (int i = 0; i < (HD + 63) / 64; ++i) {
+        const int d = lane + 64 * i;
+        if (d < HD) {
+          a.out[row + d] = acc[i];
+          if (a.split) stg[j * HD + d] = acc[i];
+        }
+      }
+    }
+  }
+  if (!q_ok) return;
+  if (!redo) {
+    float* out = a.out + (size_t)qp * qd + (size_t)h * HD;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const float4 v = make_float4(o[d][0] * inv, o[d][1] * inv, o[d][2] * inv, o[d][3] * inv);
+      *reinterpret_cast<float4*>(out + d * 16 + 4 * g) = v;
+      if (a.split) *reinterpret_cast<float4*>(stg + c16 * HD + d * 16 + 4 * g) = v;
+    }
   }
   if (a.split && lane < 16 * (HD / 32)) {  // (the LDS operations of a wave run in order)
     // the head's 32-element blocks of row i16: operand lane i16 + 16 gq of
@@ -555,21 +739,59 @@ Status build_rope_table(double* tab, int tokens, int hd, double theta, hipStream
   return hip_status(hipGetLastError(), "rope table launch");
 }
 
-// the matrix-core kernel's conditions (launch_attention)
+// The matrix-core kernel takes head dims 32, 64 and 128. Its GEN form takes
+// what the plain one does not: ALiBi, the window and prefix masks, and rings
+// shorter than a 64-key tile (whose multiplicities change within one). ALiBi
+// with the sigmoid has no common factor per ring row and stays on
+// k_attention.
 static bool attention_fast(const AttnArgs& a) {
-  return (a.mask == 1 || a.mask == 2) && !a.alibi && a.msl >= kKT && a.msl >= a.seq &&
-         (a.hd == 32 || a.hd == 64 || a.hd == 128) && a.seq > 0 && a.tokens % a.seq == 0;
+  return (a.hd == 32 || a.hd == 64 || a.hd == 128) && a.msl >= a.seq && a.seq > 0 &&
+         a.tokens % a.seq == 0 && !(a.alibi && a.sigmoid);
+}
+
+static bool attention_general(const AttnArgs& a) {
+  return a.alibi || (a.mask != 1 && a.mask != 2) || a.msl < 64;
 }
 
 bool attention_writes_split(const AttnArgs& a) {
   return attention_fast(a) && (a.heads * a.hd) % 256 == 0 && a.seq % 16 == 0;
 }
 
+template <int HD, bool SIG, bool GEN, int WAVES>
+static void attn_launch(const AttnArgs& a, hipStream_t st) {
+  const int qblocks = (a.seq + 16 * WAVES - 1) / (16 * WAVES);
+  const dim3 grid((unsigned)(a.tokens / a.seq * qblocks), (unsigned)a.heads);
+  k_attn_mfma<HD, SIG, GEN, WAVES><<<grid, 64 * WAVES, 0, st>>>(a, qblocks);
+}
+
+template <int HD, bool GEN>
+static void attn_waves_of(const AttnArgs& a, hipStream_t st) {
+  constexpr int most = HD <= 64 ? 16 : 8;
+  if (a.sigmoid) return attn_launch<HD, true, GEN, most>(a, st);
+  const auto groups = [&](int waves) {
+    return (int64_t)(a.tokens / a.seq) * a.heads * ((a.seq + 16 * waves - 1) / (16 * waves));
+  };
+  // The widest workgroup (each K/V tile staged once for more queries) that
+  // still reaches three quarters of the 256 CUs, else 4 waves, one per SIMD.
+  // Whole layers, us at 16 / 8 / 4 waves, head dim 64: 8 x 512 tokens, 16
+  // heads (256, 512, 1024 workgroups) 115 / 118 / 135; 3 x 701, 12 heads with
+  // ALiBi (108, 216, 396) 166 / 134 / 151; 1 x 1024, 16 heads (64, 128, 256)
+  // 113 / 101 / 94; 2 x 300, 8 heads (32, 48, 80) 77 / 71 / 68.
+  constexpr int64_t kFill = 192;
+  if (groups(most) >= kFill) return attn_launch<HD, false, GEN, most>(a, st);
+  if (most > 8 && groups(8) >= kFill) return attn_launch<HD, false, GEN, 8>(a, st);
+  attn_launch<HD, false, GEN, 4>(a, st);
+}
+
+template <int HD>
+static void attn_hd(const AttnArgs& a, hipStream_t st) {
+  if (attention_general(a)) attn_waves_of<HD, true>(a, st);
+  else attn_waves_of<HD, false>(a, st);
+}
+
 Status launch_attention(const AttnArgs& a, hipStream_t st) {
   if (a.hd > 64 * kMaxHdPerLane || a.hd % 4 != 0)
     return Status::err(kUnsupported, "attention: head_dim must be a multiple of 4 and <= 256");
-  // the tile multiplicity update assumes at most one multiple of msl per
-  // 64-key tile, hence msl >= 64
   const bool fast = attention_fast(a);
   if (a.split && (!attention_writes_split(a) || a.split_mpad < a.tokens || a.split_mpad % 16 != 0))
     return Status::err(kInvalid, "attention: the output split needs the matrix-core path, "
@@ -580,23 +802,10 @@ Status launch_attention(const AttnArgs& a, hipStream_t st) {
     WV_HIP(hipGetLastError());
   }
   if (fast) {
-    const int waves = attn_waves(a.hd <= 64 ? a.hd : 128), qb_rows = 16 * waves;
-    const int qblocks = (a.seq + qb_rows - 1) / qb_rows;
-    dim3 grid((unsigned)(a.tokens / a.seq * qblocks), (unsigned)a.heads);
-    const dim3 blk(64 * waves);
     switch (a.hd) {
-    case 32:
-      if (a.sigmoid) k_attn_mfma<32, true><<<grid, blk, 0, st>>>(a, qblocks);
-      else k_attn_mfma<32, false><<<grid, blk, 0, st>>>(a, qblocks);
-      break;
-    case 64:
-      if (a.sigmoid) k_attn_mfma<64, true><<<grid, blk, 0, st>>>(a, qblocks);
-      else k_attn_mfma<64, false><<<grid, blk, 0, st>>>(a, qblocks);
-      break;
-    default:
-      if (a.sigmoid) k_attn_mfma<128, true><<<grid, blk, 0, st>>>(a, qblocks);
-      else k_attn_mfma<128, false><<<grid, blk, 0, st>>>(a, qblocks);
-      break;
+    case 32: attn_hd<32>(a, st); break;
+    case 64: attn_hd<64>(a, st); break;
+    default: attn_hd<128>(a, st); break;
     }
     return hip_status(hipGetLastError(), "attention launch");
   }
