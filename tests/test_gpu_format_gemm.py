@@ -1,0 +1,102 @@
+"""The block formats' matrix-core product at the edges of its tiles: 32 or 64
+batch rows by 32, 64 or 128 weight rows, K split over 4 or 8 waves in 32-element
+sub-blocks. Reference: the session's own dequantized weights (bit-identical
+to the oracle's, test_gpu_formats.py) times x in f64. Bound: exact codes and
+x to 2^-25, fp32 sums over K/32 sub-blocks of a wave: a few 2^-24, 2e-6 with the
+cancellation of N(0, 1) inputs."""
+import numpy as np
+import pytest
+
+from test_gpu_dense import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 16, 17]
+SUPER = {6, 7, 8, 9, 10, 17}
+
+
+def weights(rng, out, inp):
+    """Rows of different magnitudes, not centred on zero."""
+    W = rng.standard_normal((out, inp)) / np.sqrt(inp) + 0.3 / np.sqrt(inp)
+    return (W * np.exp(rng.uniform(-3, 3, (out, 1)))).astype(np.float32)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("batch,inp,out", [
+    (8, 256, 33),      # the least batch; one weight row past a tile
+    (31, 768, 64),     # 24 sub-blocks over 8 waves
+    (32, 1280, 16),    # fewer weight rows than a tile
+    (33, 512, 97),     # two 32-row blocks, ragged weight tile
+    (97, 256, 200),    # last 64-row tile half empty
+    (385, 256, 1800),  # 64 x 64 tiles, ragged on both sides
+    (200, 512, 6100),  # 64 x 128 tiles, 4 waves
+])
+def test_format_gemm_matches_f64(gpu, fmt, batch, inp, out):
+    rng = np.random.default_rng(fmt * 1000 + batch + out)
+    if fmt not in SUPER:
+        inp += 96  # a number of sub-blocks that no wave count divides
+    s = gpu.FormatDenseSession(batch, inp, out, gpu.LINEAR, fmt, W=weights(rng, out, inp))
+    x = rng.standard_normal((batch, inp)).astype(np.float32)
+    x *= np.exp(rng.uniform(-6, 6, (batch, 1))).astype(np.float32)
+    y, _ = s.execute(x)
+    W = s.export_f32().astype(np.float64)
+    s.close()
+    want = x.astype(np.float64) @ W.T
+    # every batch row and every weight row by itself, against its own scale
+    scale = np.abs(x).astype(np.float64) @ np.abs(W).T
+    assert np.max(np.abs(y - want) / scale) <= 1e-6
+    assert rel_l2(y, want) <= 2e-6
+
+
+@pytest.mark.parametrize("fmt", [1, 8])
+def test_format_gemm_epilogue_and_row_runs(gpu, fmt):
+    """Bias and activation, and rows that the scratch holds in several runs
+    (the allocation-free execute has 64 MiB): the same bits as one run."""
+    rng = np.random.default_rng(fmt)
+    batch, inp, out = 1000, 16384, 40
+    bias = rng.standard_normal(out)
+    s = gpu.FormatDenseSession(batch, inp, out, gpu.SILU, fmt, W=weights(rng, out, inp), bias=bias)
+    x = rng.standard_normal((batch, inp)).astype(np.float32)
+    pre, post = s.execute(x)
+    W = s.export_f32().astype(np.float64)
+    z = (x.astype(np.float64) @ W.T + bias).astype(np.float32)
+    assert rel_l2(pre, z) <= 2e-6
+    assert rel_l2(post, pre / (1 + np.exp(-pre.astype(np.float64)))) <= 1e-6
+    h = gpu.Hip()
+    dx, dp, dq = h.upload(x), h.malloc(pre.nbytes), h.malloc(pre.nbytes)
+    s.execute_noalloc(batch, dx, dp, dq)
+    h.sync()
+    assert np.array_equal(h.download(dp, pre.shape), pre)
+    assert np.array_equal(h.download(dq, pre.shape), post)
+    for p in (dx, dp, dq):
+        h.free(p)
+    s.close()
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_format_gemm_non_finite_inputs(gpu, fmt):
+    """A row of x with an infinity, a NaN or values near the f32 maximum (whose
+    bf16 terms overflow) gives the dequantized product's result there and
+    leaves the other rows alone."""
+    rng = np.random.default_rng(fmt + 50)
+    batch, inp, out = 40, 512, 70
+    s = gpu.FormatDenseSession(batch, inp, out, gpu.LINEAR, fmt, W=weights(rng, out, inp))
+    x = rng.standard_normal((batch, inp)).astype(np.float32)
+    clean, _ = s.execute(x)
+    W = s.export_f32()
+    x[3, 17], x[9, 300], x[35, 5], x[36, 40] = np.inf, np.nan, -np.inf, np.finfo(np.float32).max
+    y, _ = s.execute(x)
+    s.close()
+    keep = [r for r in range(batch) if r not in (3, 9, 35, 36)]
+    assert np.array_equal(y[keep], clean[keep])
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = x.astype(np.float64) @ W.astype(np.float64).T
+    assert np.isnan(y[9]).all()
+    for r in (3, 35):
+        assert np.array_equal(np.isnan(y[r]), np.isnan(want[r]))
+        assert np.array_equal(np.isposinf(y[r]), np.isposinf(want[r]))
+    with np.errstate(over="ignore"):
+        top = want[36].astype(np.float32)  # some of these overflow
+    fits = np.isfinite(top)
+    assert rel_l2(y[36][fits] / 1e38, top[fits] / 1e38) <= 2e-6
+    assert np.array_equal(y[36][~fits], top[~fits])

@@ -208,6 +208,8 @@ welvet_status welvet_dense_mount_format(int32_t batch, int32_t in, int32_t out, 
     Status st = s->stream.create();
     if (st) st = wv::dense_build_format(in, out, act, format, W_init, blocks, blocks_len, bias,
                                         bias_len, &s->layer, s->stream.s);
+    if (st) st = wv::dense_prepare_rows(&s->layer, batch, s->stream.s);
+    if (st) st = wv::ensure_split(&s->ws, wv::dense_workspace_bytes(s->layer, batch));
     if (st) st = s->x.alloc((size_t)batch * in * sizeof(float));
     if (st) st = s->pre.alloc((size_t)batch * out * sizeof(float));
     if (st) st = s->post.alloc((size_t)batch * out * sizeof(float));

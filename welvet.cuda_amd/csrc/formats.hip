@@ -935,91 +935,600 @@ __global__ __launch_bounds__(64 * WAVES) void k_fmt_gemv(FmtArgs a) {
   }
 }
 
-// Batches of 2 rows and more on the matrix cores, each weight decoded once
-// for up to 16 batch rows. Workgroup (blockIdx.x, blockIdx.y): weight rows
-// r0 = 16 blockIdx.x .. +15 against batch rows j0 = 16 blockIdx.y .. +15; its
-// W waves take the groups of 4 sub-blocks (128 columns) round-robin. In a
-// group, lane (i, g) (i = lane % 16, g = lane / 16) dequantizes sub-block
-// 4q + g of weight row r0 + i to its exact f32 values (dequant_sub, the
-// oracle's arithmetic) and loads the same 32 columns of batch row j0 + i;
-// v_mfma_f32_16x16x4_f32 number m takes value m of every lane: A[i][g] the
-// weight, B[g][i] the input, so the 32 products add the group's 128 columns
-// (the four sub-blocks through the instruction's k = g). Lane (i, g) ends
-// with D[4g + r][i]: weight row r0 + 4g + r, batch row j0 + i. The waves'
-// sums are added in wave order through LDS, then the epilogue of k_fmt_gemv.
-// Batch rows from which the matrix-core kernel runs. Measured at 4096 x
-// 4096 (Q4_K, Q8_0, Q4_0, Q6_K): batch 8 14-16 us against 17-29 us for the
-// per-row kernel, batch 16 20 us against 28-52 us; at batch 2-4 the per-row
-// kernel is as fast or faster (the matrix core's 16 batch columns cost the
-// same for 2 rows as for 16).
-constexpr int kFmtMfmaBatch = 8;
+// ---- batches: the product on the bf16 matrix cores -----------------------
+// A code is an integer of at most 8 bits, exact in bf16 (the offsets of the
+// symmetric formats removed), and x is split into three bf16 terms (2^-25
+// relative), so a 32-element sub-block's sum(c x) takes three matrix-core
+// products per 16 elements and is as exact as fp32; the sub-block's scale is then applied
+// once to that sum in f32: y += d * sum(c x) + off * sum(x), off the
+// format's minimum with the code's centre (0 for the symmetric formats).
+// Formats with a scale per 16 elements (Q2_K, Q3_K, Q6_K) do so per half.
+//
+// v_mfma_f32_32x32x16_bf16: the A operand is x (lane l: batch row l % 32,
+// elements 8 (l / 32) .. + 7 of the 16), the B operand the weights (lane l:
+// weight row l % 32, the same elements), so that D's column, its lane's own,
+// is the weight row: the scale is one register per lane, and the lane that
+// decodes a weight row also holds its scale.
+//
+// k_fmt_split writes the terms in operand order, once per call: per 32 batch
+// rows and sub-block 6 KB (term, 16-element half, lane, 16 bytes). For the
+// affine formats a seventh operand follows: the sum of x over 16-element half
+// l / 32, as three terms in the elements s1 s1 s2 s1 s2 s3 0 0, which one more
+// product multiplies with the offset's o1 o2 o1 o3 o2 o1 0 0 (the six products
+// down to 2^-24 of off * sum(x)).
+//
+// k_fmt_gemm<TM, TN, W>: a workgroup owns 32 TM batch rows x 32 TN weight
+// rows; its W waves take W ranges of the sub-blocks and all of the tile, so
+// no operand is shared between waves: codes and terms go from memory to
+// registers, with no LDS and no barrier until the waves' sums are added at the
+// end (in wave order). The smaller tiles load one sub-block ahead; 2 x 4 has
+// no registers for that (128 of 256 hold sums) and leaves it to the second
+// wave of the SIMD. The weights are read from an interleaved copy, whose loads
+// are contiguous (row-major, a load touches 32 rows' lines: 80 instead of 62 us).
+// 4096 x 4096, 512 rows, Q8_0: 455 us on fp32 matrix products that decoded every
+// weight once per 16 batch rows, now 62 us with the split; 512 more rows take
+// 53 us (970 TFLOP/s of bf16 products, where a plain bf16 product of torch
+// reaches 1290). The products bound it: with a third of them it takes 46 us;
+// without the loads of x 60, of the weights 63.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
-template <int FMT, int W>
-__global__ __launch_bounds__(64 * W) void k_fmt_mfma(FmtArgs a, int batch) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & 15, g = lane >> 4;
-  const int r0 = blockIdx.x * 16, j0 = blockIdx.y * 16;
-  const int row = r0 + i;  // < rpad, a multiple of 16: in bounds
-  const bool xlive = j0 + i < batch;
-  const float* __restrict__ xr = a.x + (size_t)(xlive ? j0 + i : 0) * a.x_stride;
-  const int groups = (a.nsub + 3) / 4;
-  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-  for (int q = wave; q < groups; q += W) {
-    const int t = 4 * q + g;
-    float w[32], xv[32];
-    if (t < a.nsub) {
-      dequant_sub<FMT>(a, row, t, w);
+constexpr bool fmt_halves(int fmt) { return fmt == kQ2_K || fmt == kQ3_K || fmt == kQ6_K; }
+// bytes of the super-block header that holds the scales, if the format has one
+constexpr int fmt_header(int fmt) {
+  return fmt == kQ4_K || fmt == kQ5_K || fmt == kQ3_K ? 16 : fmt == kIQ4_XS ? 8 : 0;
+}
+constexpr bool fmt_affine(int fmt) {
+  return fmt == kQ4_1 || fmt == kQ5_1 || fmt == kQ2_K || fmt == kQ4_K || fmt == kQ5_K;
+}
+// operand bytes of 32 batch rows x 32 elements
+constexpr int fmt_split_bytes(bool affine) { return affine ? 7168 : 6144; }
+
+// v as three bf16 terms, each rounding the remainder of those before it.
+__device__ __forceinline__ void fmt_terms(float v, __bf16 (&t)[3]) {
 #pragma unroll
-      for (int e = 0; e < 32; e += 4) {
-        const float4 v = xlive ? *reinterpret_cast<const float4*>(xr + 32 * (size_t)t + e)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-        xv[e] = v.x, xv[e + 1] = v.y, xv[e + 2] = v.z, xv[e + 3] = v.w;
+  for (int k = 0; k < 3; ++k) {
+    t[k] = (__bf16)v;
+    v -= (float)t[k];
+  }
+}
+
+// One workgroup per 32 batch rows x 128 columns, staged in LDS with
+// row-contiguous loads, then one wave per sub-block: lane l holds elements 16 s +
+// 8 (l / 32) + j of row l % 32. Rows at and above `batch` are zeros.
+template <bool AFFINE>
+__global__ __launch_bounds__(kThreads) void k_fmt_split(const float* __restrict__ x, int x_stride,
+                                                        int batch, int nsub,
+                                                        uint8_t* __restrict__ xs) {
+  constexpr int kPitch = 132;  // floats: 16-byte rows, 4 banks apart
+  __shared__ __attribute__((aligned(16))) float stage[32 * kPitch];
+  const int cols = 32 * nsub;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = threadIdx.x + kThreads * k, r = i >> 5, c = 4 * (i & 31);
+    const int row = blockIdx.y * 32 + r, gc = blockIdx.x * 128 + c;
+    const bool live = row < batch && gc < cols;
+    const v4f v = *reinterpret_cast<const v4f*>(x + (size_t)(row < batch ? row : 0) * x_stride +
+                                                (gc < cols ? gc : 0));
+    *reinterpret_cast<v4f*>(stage + r * kPitch + c) = live ? v : v4f{0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, t = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  if (t >= nsub) return;  // wave-uniform
+  const int half = lane >> 5;
+  const float* src = stage + (lane & 31) * kPitch + 32 * (threadIdx.x >> 6) + 8 * half;
+  const size_t unit = (size_t)blockIdx.y * nsub + t;
+  uint8_t* dst = xs + unit * fmt_split_bytes(AFFINE) + lane * 16;
+  float sum[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const v4f lo = *reinterpret_cast<const v4f*>(src + 16 * s);
+    const v4f hi = *reinterpret_cast<const v4f*>(src + 16 * s + 4);
+    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    sum[s] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum[s] += v[j];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      bf16x8 c;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        c[j] = (__bf16)v[j];
+        v[j] -= (float)c[j];
       }
-    } else {  // past the last sub-block (cols not a multiple of 128)
-#pragma unroll
-      for (int e = 0; e < 32; ++e) w[e] = xv[e] = 0.0f;
+      *reinterpret_cast<bf16x8*>(dst + (2 * k + s) * 1024) = c;
     }
-    // every lane is active from here (the matrix core reads all 64)
+    if constexpr (AFFINE) sum[s] += __shfl_xor(sum[s], 32, 64);
+  }
+  if constexpr (AFFINE) {
+    __bf16 u[3];
+    fmt_terms(half == 0 ? sum[0] : sum[1], u);
+    const __bf16 z = (__bf16)0.0f;
+    const bf16x8 c = {u[0], u[0], u[1], u[0], u[1], u[2], z, z};
+    *reinterpret_cast<bf16x8*>(dst + 6 * 1024) = c;
+  }
+}
+
+// What lane (row, half) loads of one sub-block: the code bytes of its 2 x 8
+// elements (Q2_K, Q3_K: all 8 bytes, whose fields it picks), the high bits
+// and the scales.
+struct FmtRaw {
+  uint32_t w[4], h0, h1, s[4], e;
+};
+
+// Where a row's records lie: sub-block t of row r is record at(r) + t * step
+// of each array (super-blocks: at8(r) + t / 8 * step). Row-major, or
+// interleaved by 32 rows (FmtArgs::interleaved), so that a wave's load of one
+// sub-block of 32 rows is contiguous.
+struct FmtRow {
+  size_t sub, super;
+  int step;
+};
+
+__device__ __forceinline__ FmtRow fmt_row(const FmtArgs& a, int row) {
+  FmtRow r;
+  const size_t rb = row / 32, i = row % 32, ns = a.nsub / 8;
+  r.sub = a.interleaved ? rb * a.nsub * 32 + i : (size_t)row * a.nsub;
+  r.super = a.interleaved ? rb * ns * 32 + i : (size_t)row * ns;
+  r.step = a.interleaved ? 32 : 1;
+  return r;
+}
+
+// OCT: of the lane's 8 elements 8 o .. + 7 alone (o = 0..3); else half o (0, 1).
+template <int FMT, bool OCT = false>
+__device__ __forceinline__ void fmt_load(const FmtArgs& a, const FmtRow& row, int t, int o, FmtRaw& r) {
+  constexpr FmtGeom G = fmt_geom(FMT);
+  const size_t sub = row.sub + (size_t)(t * row.step), super = row.super + (size_t)((t >> 3) * row.step);
+  const uint8_t* q = a.q + sub * G.qb + (G.qb == 8 ? 0 : G.qb == 16 ? 8 * (o & 1) : 8 * o);
+  const uint2 w = *reinterpret_cast<const uint2*>(q);
+  r.w[0] = w.x, r.w[1] = w.y;
+  if constexpr (FMT == kQ8_0 && !OCT) {
+    const uint2 w2 = *reinterpret_cast<const uint2*>(q + 16);
+    r.w[2] = w2.x, r.w[3] = w2.y;
+  }
+  if constexpr (G.hb >= 4) r.h0 = *reinterpret_cast<const uint32_t*>(a.h + sub * G.hb);
+  if constexpr (G.hb == 8) r.h1 = *reinterpret_cast<const uint32_t*>(a.h + sub * G.hb + 4);
+  if constexpr (fmt_header(FMT) == 16) {
+    const uint4 v = *reinterpret_cast<const uint4*>(a.s + super * 16);
+    r.s[0] = v.x, r.s[1] = v.y, r.s[2] = v.z, r.s[3] = v.w;
+  } else if constexpr (fmt_header(FMT) == 8) {
+    const uint2 v = *reinterpret_cast<const uint2*>(a.s + super * 8);
+    r.s[0] = v.x, r.s[1] = v.y;
+  } else if constexpr (G.sb == 4) {
+    r.s[0] = *reinterpret_cast<const uint32_t*>(a.s + sub * 4);
+  } else {
+    r.s[0] = *reinterpret_cast<const uint16_t*>(a.s + sub * 2);
+  }
+  if constexpr (G.eb == 2) r.e = *reinterpret_cast<const uint16_t*>(a.e + super * 2);
+  if constexpr (G.eb == 4) r.e = *reinterpret_cast<const uint32_t*>(a.e + super * 4);
+}
+
+// The interleaved copy of one array: records of `bytes` (2, 4, 8, 16 or 32),
+// n per row, from [row][n] to [row / 32][n][row % 32]; rows past the source
+// are zeros. One thread per 2 bytes, the destination's neighbours in turn.
+__global__ __launch_bounds__(kThreads) void k_fmt_interleave(const uint16_t* __restrict__ src,
+                                                             uint16_t* __restrict__ dst, int rows,
+                                                             int n, int half_words, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= total) return;
+  const int b = (int)(i % half_words);
+  const int64_t rec = i / half_words;
+  const int r32 = (int)(rec % 32);
+  const int64_t u = rec / 32;
+  const int t = (int)(u % n);
+  const int64_t row = u / n * 32 + r32;
+  dst[i] = row < rows ? src[(row * n + t) * half_words + b] : (uint16_t)0;
+}
+
+// Codes as bf16: centred, times a power of two (fmt_unit) that puts them at
+// the top of a signed byte.
+template <int FMT>
+constexpr float fmt_unit() {
+  return FMT == kQ4_0 || FMT == kQ4_1 || FMT == kQ4_K   ? 1.0f / 16
+         : FMT == kQ5_0 || FMT == kQ5_1 || FMT == kQ5_K ? 1.0f / 8
+         : FMT == kQ6_K                                 ? 1.0f / 4
+         : FMT == kQ3_K                                 ? 1.0f / 32
+         : FMT == kQ2_K                                 ? 1.0f / 64
+                                                        : 1.0f;
+}
+
+// 8 consecutive elements 8 o .. 8 o + 7 (o = 0..3) of a sub-block: w their
+// code bytes (Q2_K, Q3_K: the sub-block's 8 bytes).
+template <int FMT>
+__device__ __forceinline__ bf16x8 fmt_codes8(const uint32_t (&w)[2], uint32_t h0, uint32_t h1, int o) {
+  uint32_t b[2];
 #pragma unroll
-    for (int m = 0; m < 32; ++m) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[m], xv[m], acc, 0, 0, 0);
+  for (int d = 0; d < 2; ++d) {
+    if constexpr (FMT == kQ8_0) {
+      b[d] = w[d];
+    } else if constexpr (FMT == kIQ4_NL || FMT == kIQ4_XS) {
+      b[d] = iq4_lookup((w[d] >> (4 * (o >> 1))) & 0x0F0F0F0Fu) ^ 0x80808080u;
+    } else if constexpr (FMT == kQ2_K) {
+      b[d] = (((w[d] >> (2 * o)) & 0x03030303u) << 6) ^ 0x80808080u;
+    } else if constexpr (FMT == kQ3_K) {
+      const uint32_t hb = spread1((h0 >> (8 * o + 4 * d)) & 0xFu);
+      b[d] = ((((w[d] >> (2 * o)) & 0x03030303u) | (hb << 2)) << 5) ^ 0x80808080u;
+    } else {
+      const uint32_t n = (w[d] >> (4 * (o >> 1))) & 0x0F0F0F0Fu;
+      if constexpr (FMT == kQ6_K) {
+        const uint32_t hb = spread2(((o >> 1 ? h1 : h0) >> (16 * (o & 1) + 8 * d)) & 0xFFu);
+        b[d] = ((n | (hb << 4)) << 2) ^ 0x80808080u;
+      } else if constexpr (FMT == kQ5_0 || FMT == kQ5_1 || FMT == kQ5_K) {
+        const uint32_t hb = spread1((h0 >> (8 * o + 4 * d)) & 0xFu);
+        b[d] = ((n | (hb << 4)) << 3) ^ 0x80808080u;
+      } else {
+        b[d] = (n << 4) ^ 0x80808080u;
+      }
+    }
+  }
+  // a byte's float holds it in the upper 16 bits (8 significant bits)
+  uint32_t p[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t w1 = b[k >> 1];
+    const float lo = (float)(int8_t)(w1 >> (16 * (k & 1))), hi = (float)(int8_t)(w1 >> (16 * (k & 1) + 8));
+    p[k] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+  }
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x8, (u32x4){p[0], p[1], p[2], p[3]});
+}
+
+// Scale d of the lane's codes (per half for fmt_halves) with fmt_unit
+// folded in, and the offset that multiplies sum(x).
+template <int FMT>
+__device__ __forceinline__ void fmt_scales(const FmtRaw& r, int t, float (&d)[2], float (&off)[2]) {
+  constexpr float U = fmt_unit<FMT>();
+  off[0] = off[1] = 0.0f;
+  if constexpr (FMT == kQ8_0 || FMT == kIQ4_NL || FMT == kQ4_0 || FMT == kQ5_0) {
+    d[0] = d[1] = f16f((uint16_t)r.s[0]) * U;
+  } else if constexpr (FMT == kQ4_1 || FMT == kQ5_1) {
+    const float dd = f16f((uint16_t)r.s[0]);
+    d[0] = d[1] = dd * U;
+    off[0] = off[1] = fmaf(FMT == kQ4_1 ? 8.0f : 16.0f, dd, f16f((uint16_t)(r.s[0] >> 16)));
+  } else if constexpr (FMT == kQ4_K || FMT == kQ5_K) {
+    int sc, m;
+    scale_min_k4_regs(t & 7, r.s[1], r.s[2], r.s[3], &sc, &m);
+    const float d1 = f16f((uint16_t)r.s[0]) * (float)sc, m1 = f16f((uint16_t)(r.s[0] >> 16)) * (float)m;
+    d[0] = d[1] = d1 * U;
+    off[0] = off[1] = fmaf(FMT == kQ4_K ? 8.0f : 16.0f, d1, -m1);
+  } else if constexpr (FMT == kIQ4_XS) {
+    const int ib = t & 7;
+    const int ls = (int)(((r.s[1] >> (8 * (ib >> 1) + 4 * (ib & 1))) & 15u) |
+                         (((r.s[0] >> (16 + 2 * ib)) & 3u) << 4));
+    d[0] = d[1] = f16f((uint16_t)r.s[0]) * (float)(ls - 32);
+  } else if constexpr (FMT == kQ2_K) {
+    const float dd = f16f((uint16_t)r.e), dmin = f16f((uint16_t)(r.e >> 16));
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const float dl = dd * (float)((r.s[0] >> (8 * s)) & 15u);
+      d[s] = dl * U;
+      off[s] = fmaf(2.0f, dl, -dmin * (float)((r.s[0] >> (8 * s + 4)) & 15u));
+    }
+  } else if constexpr (FMT == kQ3_K) {
+    const float dd = f16f((uint16_t)r.s[3]);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      d[s] = dd * (float)scale_q3k_regs(2 * (t & 7) + s, r.s[0], r.s[1], r.s[2]) * U;
+  } else {
+    const float dd = f16f((uint16_t)r.e);
+    d[0] = dd * (float)(int8_t)r.s[0] * U;
+    d[1] = dd * (float)(int8_t)(r.s[0] >> 8) * U;
+  }
+}
+
+// One output over the dequantized weights, for a sum that is not finite: the
+// bf16 terms of an infinity (or of a value that rounds to one) are NaN.
+template <int FMT>
+__device__ float fmt_dot(const FmtArgs& a, int row, const float* __restrict__ x) {
+  float v = 0.0f;
+  for (int t = 0; t < a.nsub; ++t) {
+    float w[32];
+    dequant_sub<FMT>(a, row, t, w);
+#pragma unroll
+    for (int e = 0; e < 32; ++e) v = fmaf(w[e], x[32 * (size_t)t + e], v);
+  }
+  return v;
+}
+
+// The Dense epilogue of output (batch row j, weight row o).
+template <int FMT>
+__device__ __forceinline__ void fmt_store(const FmtArgs& a, int j, int o, float v) {
+  if (!(v - v == 0.0f)) v = fmt_dot<FMT>(a, o, a.x + (size_t)j * a.x_stride);
+  const size_t oi = (size_t)j * a.out_stride + o;
+  if (a.need_epi) {
+    double d = (double)v;
+    if (a.bias && o < a.bias_len) {
+      d += a.bias[o];
+      v = (float)d;
+    }
+    a.pre[oi] = v;
+    a.post[oi] = (float)act_f64(a.act, d);
+  } else {
+    a.pre[oi] = v;
+    if (a.post && a.post != a.pre) a.post[oi] = v;
+  }
+}
+
+template <int FMT, int TM, int TN, int W>
+__global__ __launch_bounds__(64 * W) void k_fmt_gemm(FmtArgs a, FmtArgs plain,
+                                                     const uint8_t* __restrict__ xs,
+                                                     int batch, int mtiles) {
+  constexpr bool HALVES = fmt_halves(FMT), AFFINE = fmt_affine(FMT);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  // workgroups are dealt round-robin to the 8 XCDs: each takes one run of
+  // tiles, all batch tiles of a weight tile in turn
+  const int tiles = gridDim.x, per = (tiles + 7) / 8;
+  const int big = tiles % 8 ? tiles % 8 : 8, x8 = blockIdx.x & 7, i8 = blockIdx.x >> 3;
+  const int tile = (x8 < big ? x8 * per : big * per + (x8 - big) * (per - 1)) + i8;
+  const int mt = tile % mtiles, n0 = tile / mtiles * 32 * TN;
+  const int mblocks = (batch + 31) / 32;
+  const int t0 = (int)((int64_t)a.nsub * wave / W), t1 = (int)((int64_t)a.nsub * (wave + 1) / W);
+  FmtRow row[TN];
+#pragma unroll
+  for (int n = 0; n < TN; ++n) {
+    const int r = n0 + 32 * n + col;
+    row[n] = fmt_row(a, r < a.rows ? r : a.rows - 1);
+  }
+  size_t unit0[TM];  // (32-row block, sub-block 0) of the terms
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int mb = mt * TM + m;
+    unit0[m] = (size_t)(mb < mblocks ? mb : mblocks - 1) * a.nsub;
+  }
+  v16f acc[TM][TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) acc[m][n] = (v16f)(0.0f);
+
+  struct Step {
+    bf16x8 x[TM][3][2];
+    bf16x8 sum[TM];
+    FmtRaw w[TN];
+  };
+  auto load = [&](int t, Step& p) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n) fmt_load<FMT>(a, row[n], t, half, p.w[n]);
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      const uint8_t* src = xs + (unit0[m] + t) * fmt_split_bytes(AFFINE) + lane * 16;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) p.x[m][k >> 1][k & 1] = *reinterpret_cast<const bf16x8*>(src + k * 1024);
+      if constexpr (AFFINE) p.sum[m] = *reinterpret_cast<const bf16x8*>(src + 6 * 1024);
+    }
+  };
+  auto compute = [&](int t, const Step& p) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      float d[2], off[2];
+      fmt_scales<FMT>(p.w[n], t, d, off);
+      constexpr int W1 = FMT == kQ8_0 ? 2 : 0;  // Q8_0: the second 8 bytes
+      const FmtRaw& f = p.w[n];
+      const bf16x8 b0 = fmt_codes8<FMT>({f.w[0], f.w[1]}, f.h0, f.h1, half);
+      const bf16x8 b1 = fmt_codes8<FMT>({f.w[W1], f.w[W1 + 1]}, f.h0, f.h1, 2 + half);
+      bf16x8 bo;
+      if constexpr (AFFINE) {
+        __bf16 u[3];
+        fmt_terms(half == 0 ? off[0] : off[1], u);
+        const __bf16 z = (__bf16)0.0f;
+        bo = bf16x8{u[0], u[1], u[0], u[2], u[1], u[0], z, z};
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        v16f d0 = (v16f)(0.0f);
+#pragma unroll
+        for (int k = 2; k >= 0; --k) d0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p.x[m][k][0], b0, d0, 0, 0, 0);
+        if constexpr (HALVES) {
+          v16f d1 = (v16f)(0.0f);
+#pragma unroll
+          for (int k = 2; k >= 0; --k) d1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p.x[m][k][1], b1, d1, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[m][n][r] = fmaf(d[1], d1[r], fmaf(d[0], d0[r], acc[m][n][r]));
+        } else {
+#pragma unroll
+          for (int k = 2; k >= 0; --k) d0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p.x[m][k][1], b1, d0, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[m][n][r] = fmaf(d[0], d0[r], acc[m][n][r]);
+        }
+        if constexpr (AFFINE) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p.sum[m], bo, acc[m][n], 0, 0, 0);
+      }
+    }
+  };
+  if constexpr (TM * TN == 8) {
+    for (int t = t0; t < t1; ++t) {
+      Step p;
+      load(t, p);
+      compute(t, p);
+    }
+  } else if (t0 < t1) {
+    Step p, q;
+    load(t0, p);
+    int t = t0;
+    // (the barriers keep the next sub-block's loads ahead of this one's products)
+    for (; t + 2 <= t1; t += 2) {
+      load(t + 1, q);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(t, p);
+      __builtin_amdgcn_sched_barrier(0);
+      load(t + 2 < t1 ? t + 2 : t + 1, p);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(t + 1, q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (t < t1) compute(t, p);
+  }
+
+  // the waves' sums of kRound 32 x 32 tiles at a time; thread i adds one
+  // (register, lane) of them in wave order
+  constexpr int kRound = TM * TN < 4 ? TM * TN : W <= 4 ? 4 : 2;
+  __shared__ float part[kRound][W][16][64];
+#pragma unroll
+  for (int c0 = 0; c0 < TM * TN; c0 += kRound) {
+    if (c0) __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kRound; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[c][wave][r][lane] = acc[(c0 + c) % TM][(c0 + c) / TM][r];
+    __syncthreads();
+    for (int i = threadIdx.x; i < kRound * 1024; i += 64 * W) {
+      const int c = i >> 10, r = (i >> 6) & 15;
+      const int tm = (c0 + c) % TM, tn = (c0 + c) / TM;
+      const int j = (mt * TM + tm) * 32 + 8 * (r >> 2) + 4 * ((i >> 5) & 1) + (r & 3);
+      const int o = n0 + 32 * tn + (i & 31);
+      if (j >= batch || o >= a.rows) continue;
+      float v = part[c][0][r][i & 63];
+#pragma unroll
+      for (int w = 1; w < W; ++w) v += part[c][w][r][i & 63];
+      fmt_store<FMT>(plain, j, o, v);
+    }
+  }
+}
+
+// At most 16 batch rows in one launch: a workgroup owns 16 weight rows and
+// all the batch rows, its W waves split the sub-blocks, x is split by the wave
+// itself (v_mfma_f32_16x16x32_bf16: lane l holds elements 8 (l / 16) .. + 7 of
+// batch row, and of weight row, l % 16; one product per term and sub-block,
+// two with the other half zeroed for fmt_halves). Bound by the latency of its
+// loads: those of `kDepth` sub-blocks are issued before the first of them is
+// used, and 16 waves make it two rounds at 4096 columns. 4096 x 4096 Q4_0 at 8
+// rows 10.2 us (13.0 on the fp32 matrix products), at 4 rows 9.6 us (11.6 with
+// every batch row streaming the weights); from row-major weights 14.9.
+template <int FMT, int W>
+__global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, int batch) {
+  constexpr bool HALVES = fmt_halves(FMT), AFFINE = fmt_affine(FMT);
+  constexpr int kDepth = 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i16 = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const FmtRow row = fmt_row(a, n0 + i16 < a.rows ? n0 + i16 : a.rows - 1);
+  const int t0 = (int)((int64_t)a.nsub * wave / W), t1 = (int)((int64_t)a.nsub * (wave + 1) / W);
+  const bool live = i16 < batch;
+  const float* src = a.x + (size_t)(live ? i16 : 0) * a.x_stride + 8 * g;
+  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+  const bf16x8 zero = (bf16x8)(__bf16)0.0f;
+
+  for (int tb = t0; tb < t1; tb += kDepth) {
+    FmtRaw raw[kDepth];
+    v4f xv[kDepth][2];
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+      const int t = tb + u < t1 ? tb + u : t1 - 1;
+      fmt_load<FMT, true>(a, row, t, g, raw[u]);
+      xv[u][0] = *reinterpret_cast<const v4f*>(src + 32 * (size_t)t);
+      xv[u][1] = *reinterpret_cast<const v4f*>(src + 32 * (size_t)t + 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+      float d[2], off[2];
+      fmt_scales<FMT>(raw[u], tb + u < t1 ? tb + u : t1 - 1, d, off);
+      // past the range: the last sub-block again, times 0 (a branch here would
+      // take the loads along)
+      const float on = tb + u < t1 ? 1.0f : 0.0f;
+      d[0] *= on, d[1] *= on, off[0] *= on, off[1] *= on;
+      const bf16x8 b = fmt_codes8<FMT>({raw[u].w[0], raw[u].w[1]}, raw[u].h0, raw[u].h1, g);
+      const bf16x8 b0 = HALVES && g >= 2 ? zero : b, b1 = g < 2 ? zero : b;
+      bf16x8 bo = zero;
+      if constexpr (AFFINE) {
+        __bf16 c[3];
+        fmt_terms(g < 2 ? off[0] : off[1], c);
+        if ((g & 1) == 0) bo = bf16x8{c[0], c[1], c[0], c[2], c[1], c[0], zero[0], zero[0]};
+      }
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = live ? xv[u][j >> 2][j & 3] : 0.0f;
+      float sum = 0.0f;
+      if constexpr (AFFINE) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum += v[j];
+        sum += __shfl_xor(sum, 16, 64);
+      }
+      bf16x8 x[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x[k][j] = (__bf16)v[j];
+          v[j] -= (float)x[k][j];
+        }
+      v4f d0 = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 2; k >= 0; --k) d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[k], b0, d0, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = fmaf(d[0], d0[r], acc[r]);
+      if constexpr (HALVES) {
+        d0 = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 2; k >= 0; --k) d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[k], b1, d0, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = fmaf(d[1], d0[r], acc[r]);
+      }
+      if constexpr (AFFINE) {
+        __bf16 c[3];
+        fmt_terms(sum, c);
+        const bf16x8 xo = {c[0], c[0], c[1], c[0], c[1], c[2], zero[0], zero[0]};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xo, bo, acc, 0, 0, 0);
+      }
+    }
   }
 
   __shared__ v4f part[W][64];
   part[wave][lane] = acc;
   __syncthreads();
-  if (wave != 0) return;
-  v4f y = part[0][lane];
+  // thread: (batch row, weight row) with the weight rows side by side; D's
+  // element r of lane (column i, group g) is batch row 4 g + r, weight row i
+  for (int i = threadIdx.x; i < 256; i += 64 * W) {
+    const int j = i >> 4, o = n0 + (i & 15);
+    if (j >= batch || o >= a.rows) continue;
+    const int l = (j >> 2) * 16 + (i & 15), r = j & 3;
+    float v = part[0][l][r];
 #pragma unroll
-  for (int w = 1; w < W; ++w) y += part[w][lane];
-  const int j = j0 + i;
-  if (j >= batch) return;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int o = r0 + 4 * g + r;
-    if (o >= a.rows) break;
-    const size_t oi = (size_t)j * a.out_stride + o;
-    float v = y[r];
-    if (a.need_epi) {
-      double d = (double)v;
-      if (a.bias && o < a.bias_len) {
-        d += a.bias[o];
-        v = (float)d;
-      }
-      a.pre[oi] = v;
-      a.post[oi] = (float)act_f64(a.act, d);
-    } else {
-      a.pre[oi] = v;
-      if (a.post && a.post != a.pre) a.post[oi] = v;
-    }
+    for (int w = 1; w < W; ++w) v += part[w][l][r];
+    fmt_store<FMT>(plain, j, o, v);
   }
 }
 
+// The weights as the matrix-core tiles read them: interleaved if they are.
+FmtArgs tile_weights(FmtArgs a, const FmtTiles& f) {
+  if (f.q) a.q = f.q, a.h = f.h, a.s = f.s, a.e = f.e;
+  a.interleaved = f.q != nullptr;
+  return a;
+}
+
+template <int FMT, int W>
+Status rows_t(const FmtArgs& a, const FmtTiles& f, int batch, hipStream_t st) {
+  k_fmt_rows<FMT, W><<<(unsigned)((a.rows + 15) / 16), 64 * W, 0, st>>>(tile_weights(a, f), a, batch);
+  return hip_status(hipGetLastError(), "format rows launch");
+}
+
+template <int FMT, int TM, int TN, int W>
+Status gemm_t(const FmtArgs& a, const FmtTiles& f, int batch, const uint8_t* xs, hipStream_t st) {
+  const FmtArgs w = tile_weights(a, f);
+  const int mtiles = (batch + 32 * TM - 1) / (32 * TM), ntiles = (a.rows + 32 * TN - 1) / (32 * TN);
+  k_fmt_gemm<FMT, TM, TN, W><<<(unsigned)(mtiles * ntiles), 64 * W, 0, st>>>(w, a, xs, batch, mtiles);
+  return hip_status(hipGetLastError(), "format gemm launch");
+}
+
 template <int FMT>
-Status mfma_f(const FmtArgs& a, int batch, hipStream_t st) {
-  constexpr int W = 8;
-  const dim3 grid((unsigned)((a.rows + 15) / 16), (unsigned)((batch + 15) / 16));
-  k_fmt_mfma<FMT, W><<<grid, 64 * W, 0, st>>>(a, batch);
-  return hip_status(hipGetLastError(), "format matrix-core gemv launch");
+Status gemm_f(const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws, hipStream_t st) {
+  const int mblocks = (batch + 31) / 32;
+  const dim3 grid((unsigned)((a.nsub + 3) / 4), (unsigned)mblocks);
+  k_fmt_split<fmt_affine(FMT)><<<grid, kThreads, 0, st>>>(a.x, a.x_stride, batch, a.nsub, ws);
+  WV_HIP(hipGetLastError());
+  const auto tiles = [&](int tm, int tn) {
+    return (int64_t)((batch + 32 * tm - 1) / (32 * tm)) * ((a.rows + 32 * tn - 1) / (32 * tn));
+  };
+  // The largest tile (a decoded weight and a loaded term feed more products)
+  // that still reaches three quarters of the 256 CUs. 4096 x 4096 Q4_0, us at
+  // tiles 1 x 1 / 1 x 2 / 2 x 2 / 2 x 4: 64 rows 15.9 / 19.0 / 31.9 / 49.0, 128
+  // rows 26.6 / 22.1 / 34.1 / 49.3, 256 rows 50.4 / 39.7 / 40.1 / 52.5, 512 rows
+  // 114 / 75 / 74 / 62.
+  constexpr int64_t kFill = 192;
+  if (tiles(2, 4) >= kFill) return gemm_t<FMT, 2, 4, 8>(a, f, batch, ws, st);
+  if (tiles(2, 2) >= kFill) return gemm_t<FMT, 2, 2, 8>(a, f, batch, ws, st);
+  if (tiles(1, 2) >= kFill) return gemm_t<FMT, 1, 2, 8>(a, f, batch, ws, st);
+  return gemm_t<FMT, 1, 1, 8>(a, f, batch, ws, st);
 }
 
 template <int FMT, int R>
@@ -1034,8 +1543,22 @@ Status gemv_w(const FmtArgs& a, int batch, int waves, hipStream_t st) {
 }
 
 template <int FMT>
-Status gemv_f(const FmtArgs& a, int batch, hipStream_t st) {
-  if (batch >= kFmtMfmaBatch) return mfma_f<FMT>(a, batch, st);
+Status gemv_f(const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws, size_t ws_bytes,
+              hipStream_t st) {
+  if (batch >= format_rows_batch(FMT) && batch <= 16) return rows_t<FMT, 16>(a, f, batch, st);
+  if (batch > 16 && ws) {
+    // as many rows at a time as the workspace holds terms of
+    const size_t unit = (size_t)a.nsub * fmt_split_bytes(fmt_affine(FMT));
+    const int64_t rows = (int64_t)(ws_bytes / unit) * 32;
+    for (int64_t j = 0; rows > 0 && j < batch; j += rows) {
+      FmtArgs c = a;
+      c.x = a.x + (size_t)j * a.x_stride;
+      c.pre = a.pre + (size_t)j * a.out_stride;
+      c.post = a.post ? a.post + (size_t)j * a.out_stride : nullptr;
+      WV_TRY(gemm_f<FMT>(c, f, (int)(batch - j < rows ? batch - j : rows), ws, st));
+    }
+    if (rows > 0) return Status::ok();
+  }
   // one wave per 64-sub-block chunk up to 4; then rows per group so that the
   // grid has >= 8 waves per CU when it can
   const int chunks = (a.nsub + 63) / 64;
@@ -1132,23 +1655,62 @@ Status format_dequant(int fmt, const FmtArgs& a, int rows, float* out, hipStream
   }
 }
 
-Status launch_format_gemv(int fmt, const FmtArgs& a, int batch, hipStream_t st) {
+size_t format_interleaved_bytes(int fmt, int rows, int nsub) {
+  const FmtGeom G = fmt_geom(fmt);
+  const size_t subs = (size_t)round_up(rows, 32) * nsub;
+  // (each array at a 256-byte boundary)
+  return round_up(subs * G.qb, 256) + round_up(subs * G.hb, 256) + round_up(subs * G.sb, 256) +
+         round_up(subs / 8 * G.eb, 256);
+}
+
+Status format_interleave(int fmt, const FmtArgs& a, uint8_t* buf, int rpad, FmtTiles* f,
+                         hipStream_t st) {
+  const FmtGeom G = fmt_geom(fmt);
+  if (G.qk == 0 || !buf || !f) return Status::err(kInvalid, "format interleave: bad args");
+  const int rows32 = (int)round_up(a.rows, 32);
+  const auto array = [&](const uint8_t* src, int n, int bytes, const uint8_t** out) -> Status {
+    *out = nullptr;
+    if (bytes == 0) return Status::ok();
+    const int64_t total = (int64_t)rows32 * n * (bytes / 2);
+    k_fmt_interleave<<<(unsigned)((total + kThreads - 1) / kThreads), kThreads, 0, st>>>(
+        reinterpret_cast<const uint16_t*>(src), reinterpret_cast<uint16_t*>(buf), rpad, n, bytes / 2,
+        total);
+    *out = buf;
+    buf += round_up((int64_t)total * 2, 256);
+    return hip_status(hipGetLastError(), "format interleave launch");
+  };
+  WV_TRY(array(a.q, a.nsub, G.qb, &f->q));
+  WV_TRY(array(a.h, a.nsub, G.hb, &f->h));
+  // headers are one record per super-block
+  const int hd = fmt_header(fmt);
+  WV_TRY(array(a.s, hd ? a.nsub / 8 : a.nsub, hd ? hd : G.sb, &f->s));
+  return array(a.e, a.nsub / 8, G.eb, &f->e);
+}
+
+size_t format_ws_bytes(int nsub, int batch) {
+  if (batch <= 16) return 0;
+  const size_t n = (size_t)((batch + 31) / 32) * nsub * fmt_split_bytes(true);
+  return n < kFmtWsBytes ? n : kFmtWsBytes;
+}
+
+Status launch_format_gemv(int fmt, const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws,
+                          size_t ws_bytes, hipStream_t st) {
   if (a.nsub <= 0 || a.rows <= 0 || batch <= 0) return Status::err(kInvalid, "format gemv: shape");
   if ((reinterpret_cast<uintptr_t>(a.x) & 15u) || (a.x_stride % 4))
     return Status::err(kInvalid, "format gemv: x must be 16-byte aligned with a stride of 4k");
   switch (fmt) {
-  case kQ8_0: return gemv_f<kQ8_0>(a, batch, st);
-  case kQ4_0: return gemv_f<kQ4_0>(a, batch, st);
-  case kQ4_1: return gemv_f<kQ4_1>(a, batch, st);
-  case kQ5_0: return gemv_f<kQ5_0>(a, batch, st);
-  case kQ5_1: return gemv_f<kQ5_1>(a, batch, st);
-  case kQ2_K: return gemv_f<kQ2_K>(a, batch, st);
-  case kQ3_K: return gemv_f<kQ3_K>(a, batch, st);
-  case kQ4_K: return gemv_f<kQ4_K>(a, batch, st);
-  case kQ5_K: return gemv_f<kQ5_K>(a, batch, st);
-  case kQ6_K: return gemv_f<kQ6_K>(a, batch, st);
-  case kIQ4_NL: return gemv_f<kIQ4_NL>(a, batch, st);
-  case kIQ4_XS: return gemv_f<kIQ4_XS>(a, batch, st);
+  case kQ8_0: return gemv_f<kQ8_0>(a, f, batch, ws, ws_bytes, st);
+  case kQ4_0: return gemv_f<kQ4_0>(a, f, batch, ws, ws_bytes, st);
+  case kQ4_1: return gemv_f<kQ4_1>(a, f, batch, ws, ws_bytes, st);
+  case kQ5_0: return gemv_f<kQ5_0>(a, f, batch, ws, ws_bytes, st);
+  case kQ5_1: return gemv_f<kQ5_1>(a, f, batch, ws, ws_bytes, st);
+  case kQ2_K: return gemv_f<kQ2_K>(a, f, batch, ws, ws_bytes, st);
+  case kQ3_K: return gemv_f<kQ3_K>(a, f, batch, ws, ws_bytes, st);
+  case kQ4_K: return gemv_f<kQ4_K>(a, f, batch, ws, ws_bytes, st);
+  case kQ5_K: return gemv_f<kQ5_K>(a, f, batch, ws, ws_bytes, st);
+  case kQ6_K: return gemv_f<kQ6_K>(a, f, batch, ws, ws_bytes, st);
+  case kIQ4_NL: return gemv_f<kIQ4_NL>(a, f, batch, ws, ws_bytes, st);
+  case kIQ4_XS: return gemv_f<kIQ4_XS>(a, f, batch, ws, ws_bytes, st);
   default: return Status::err(kGap, "gap? quant format not implemented");
   }
 }

@@ -357,6 +357,7 @@ struct FmtArgs {
   const uint8_t* h = nullptr;  // [rpad][nsub][hb]
   const uint8_t* s = nullptr;  // [rpad][nsub][sb]
   const uint8_t* e = nullptr;  // [rpad][nsub / 8][eb] (Q2_K d, dmin; Q6_K d)
+  bool interleaved = false;  // q, h, s and e are FmtTiles' arrays
   int rows = 0, cols = 0, nsub = 0;  // nsub = cols / 32
   const float* x = nullptr;
   int x_stride = 0;
@@ -375,8 +376,31 @@ Status format_quantize(int fmt, const float* W, int64_t n, uint8_t* out, hipStre
 Status format_relayout(int fmt, const FmtArgs& a, const uint8_t* blocks, int rows, hipStream_t st);
 // The resident arrays -> f32 [rows][cols] (the format's dequantization).
 Status format_dequant(int fmt, const FmtArgs& a, int rows, float* out, hipStream_t st);
+// A copy of the arrays with the records of 32 rows side by side
+// ([row / 32][sub-block][row % 32]), which the matrix-core product reads with
+// contiguous loads: into buf (format_interleaved_bytes). rpad: rows of the
+// source arrays.
+struct FmtTiles {
+  const uint8_t *q = nullptr, *h = nullptr, *s = nullptr, *e = nullptr;
+};
+size_t format_interleaved_bytes(int fmt, int rows, int nsub);
+Status format_interleave(int fmt, const FmtArgs& a, uint8_t* buf, int rpad, FmtTiles* f,
+                         hipStream_t st);
+// Batch rows from which the matrix cores take the product. 4096 x 4096 at 4 and
+// 6 rows, us, the per-row kernel against the matrix cores: Q8_0 16.3 / 10.0 and
+// 21.7 / 10.4, Q4_0 11.6 / 9.8 and 13.8 / 10.1, Q4_1 10.1 / 11.6 and 13.8 /
+// 11.9, Q2_K 11.5 / 13.6 and 14.3 / 14.0 (the others like Q4_0).
+constexpr int format_rows_batch(int fmt) {
+  return fmt == kQ2_K ? 6 : fmt == kQ4_1 || fmt == kQ5_1 ? 5 : 4;
+}
 // y = W x for every one of `batch` rows of x (a.x, a.x_stride), with the Dense
-// epilogue into a.pre / a.post.
-Status launch_format_gemv(int fmt, const FmtArgs& a, int batch, hipStream_t st);
+// epilogue into a.pre / a.post. f: the interleaved copy, if there is one. ws:
+// scratch for the product above 16 rows (format_ws_bytes, at most kFmtWsBytes,
+// beyond which it takes the rows in several runs); without it every batch
+// row streams the weights there.
+constexpr size_t kFmtWsBytes = 64ull << 20;
+size_t format_ws_bytes(int nsub, int batch);
+Status launch_format_gemv(int fmt, const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws,
+                          size_t ws_bytes, hipStream_t st);
 
 }  // namespace wv

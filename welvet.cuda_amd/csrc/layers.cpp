@@ -208,7 +208,7 @@ Status dense_export_f32(const DenseLayer& L, float* w, hipStream_t st) {
 }
 
 static Status format_forward(const DenseLayer& L, int batch, const float* x, float* pre,
-                             float* post, hipStream_t st) {
+                             float* post, Workspace* ws, hipStream_t st) {
   FmtArgs a = format_args(L);
   a.x = x;
   a.x_stride = L.in;
@@ -219,7 +219,9 @@ static Status format_forward(const DenseLayer& L, int batch, const float* x, flo
   a.need_epi = L.need_epi();
   a.bias = L.bias_dev.as<const double>();
   a.bias_len = L.bias_len;
-  return launch_format_gemv(L.format, a, batch, st);
+  if (ws) WV_TRY(ensure_split(ws, format_ws_bytes(L.fw.nsub, batch)));
+  return launch_format_gemv(L.format, a, L.fw.tiles, batch, ws ? split_buf(ws) : nullptr,
+                            ws ? ws->b.bytes : 0, st);
 }
 
 int gemv_batch_limit() { return 1 << 30; }
@@ -291,7 +293,13 @@ static Status build_frag(DenseLayer* L, hipStream_t st) {
 }
 
 Status dense_prepare_rows(DenseLayer* L, int batch, hipStream_t st) {
-  if (L->format) return Status::ok();
+  if (L->format) {
+    FormatWeights& f = L->fw;
+    if (batch < format_rows_batch(f.format) || f.il.p) return Status::ok();
+    WV_TRY(f.il.alloc(format_interleaved_bytes(f.format, f.rows, f.nsub)));
+    WV_TRY(format_interleave(f.format, format_args(*L), f.il.as<uint8_t>(), f.rpad, &f.tiles, st));
+    return hip_status(hipStreamSynchronize(st), "format interleave");
+  }
   if ((uses_split(batch) && mxg_block_m(batch) == 16) || mx_dense(*L, batch)) return build_frag(L, st);
   return Status::ok();
 }
@@ -335,7 +343,7 @@ static size_t gemm_ws_bytes(const DenseLayer& L, int batch, int mats) {
 }
 
 size_t dense_workspace_bytes(const DenseLayer& L, int batch) {
-  if (L.format) return 0;
+  if (L.format) return format_ws_bytes(L.fw.nsub, batch);
   return uses_split(batch) ? gemm_ws_bytes(L, batch, 1) : 0;
 }
 
@@ -441,8 +449,8 @@ Status dense_forward(const DenseLayer& L, int batch, const float* x, float* pre,
                      Workspace* ws, hipStream_t st) {
   if (batch <= 0 || !x || !pre) return Status::err(kInvalid, "dense forward: bad args");
   if (L.need_epi() && !post) return Status::err(kInvalid, "dense forward: post needed");
-  // packed block formats: the GEMV over every batch row
-  if (L.format) return format_forward(L, batch, x, pre, post, st);
+  // packed block formats: their own GEMV and matrix-core product
+  if (L.format) return format_forward(L, batch, x, pre, post, ws, st);
   if (mx_dense(L, batch) && L.dev.codes_frag.p && mx_vec(L, x)) {
     GemvMxArgs m = mx_args(L, x, batch);
     m.pre = pre;

@@ -56,6 +56,10 @@ struct Workspace {
 struct FormatWeights {
   int format = 0, rows = 0, cols = 0, rpad = 0, nsub = 0;
   DevBuf q, h, s, e;
+  // optional second copy, interleaved by 32 rows for the matrix-core product
+  // (built by sessions whose batch runs it), and its arrays
+  DevBuf il;
+  FmtTiles tiles;
   std::vector<uint8_t> blocks;
 };
 
