@@ -8,7 +8,8 @@
 //              (src/runtime/training.cpp:44-69). Not launched for a Linear
 //              layer without a target: there d_pre is gy, which k_bwd reads
 //              directly and stores as d_pre.
-//   k_bwd      both products, which read only d_pre, in one launch:
+//   k_bwd      both products of one or two batch rows, which read only d_pre, in
+//              one launch:
 //              * dX = W^T d_pre (kernels.cu:92-107) from the code rows the
 //                forward streams: a workgroup owns 1024 columns and a band of
 //                rows, each lane 16 consecutive columns (one 16-byte FP8 or
@@ -23,6 +24,8 @@
 //                the dX ones. The f64 product of two floats is exact, so this
 //                is bit-exact. The read-bound dX stream and the write-bound dW
 //                stream share the launch and overlap in HBM.
+//   k_dx_mfma  dX of more batch rows on the f64 matrix cores.
+//   k_outer    dW of more batch rows.
 //   k_gemvt_reduce  adds the band partials in a fixed order, rounds to f32.
 //   k_sgd      w' = f32(f64(w) - lr * f64(dW)), w the dequantized f32 weight
 //              (native_codec.cpp:1112-1128, weight_at / set_weight_at); the
@@ -42,7 +45,7 @@ constexpr int kThreads = 256;
 constexpr int kCpl = 16;                // dX columns per lane
 constexpr int kTileCols = 64 * kCpl;    // columns per dX workgroup
 constexpr int kRowsInFlight = 8;        // code rows loaded ahead per wave
-constexpr int kBatchChunk = 2;          // d_pre rows per launch
+constexpr int kStreamRows = 2;          // batch rows up to which k_bwd runs
 constexpr int kOuterRows = 4;           // dW rows per workgroup
 
 typedef float v2f __attribute__((ext_vector_type(2)));
@@ -155,11 +158,11 @@ struct OuterArgs {
 
 // dX part: workgroup `blk` of the first tiles * bands owns 1024 columns
 // (lane: 16) and a band of rows; wave w takes rows o0 + w, + 4, ..., 8 rows'
-// loads in flight at a time. d_pre rows b0 .. b0 + NB - 1. Lanes past the
+// loads in flight at a time. NB batch rows. Lanes past the
 // padded row read column 0 (never stored). The 4 waves' sums are added in
 // wave order through LDS into the band's partial row.
 template <int DT, bool BLK, int NB>
-__device__ __forceinline__ void gemvt_tile(const GemvtArgs& a, int blk, int tiles, int bands, int b0,
+__device__ __forceinline__ void gemvt_tile(const GemvtArgs& a, int blk, int tiles, int bands,
                                            double* __restrict__ part, double (*red)[NB][kTileCols]) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = blk % tiles, band = blk / tiles;
@@ -169,7 +172,7 @@ __device__ __forceinline__ void gemvt_tile(const GemvtArgs& a, int blk, int tile
   typedef typename RowCodes<DT>::T Q;
   const uint8_t* base = a.codes + (DT == kFP4 ? cc / 2 : cc);
   const ConstF32 sc = (ConstF32)a.scale;
-  const ConstF32 dp = (ConstF32)(a.dpre + (size_t)b0 * a.out);
+  const ConstF32 dp = (ConstF32)a.dpre;
   double acc[NB][kCpl];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -283,14 +286,187 @@ __device__ __forceinline__ void outer_rows(const float* __restrict__ dpre, const
 // first tiles * bands workgroups stream the codes for dX partials, the rest
 // write dW, so the read-bound and the write-bound streams overlap in HBM.
 template <int DT, bool BLK, int NB>
-__global__ __launch_bounds__(kThreads) void k_bwd(GemvtArgs a, int b0, int tiles, int bands,
+__global__ __launch_bounds__(kThreads) void k_bwd(GemvtArgs a, int tiles, int bands,
                                                   double* __restrict__ part, OuterArgs oa) {
   __shared__ double red[4][NB][kTileCols];
   const int gemvt_blocks = tiles * bands;
   if ((int)blockIdx.x < gemvt_blocks) {
-    gemvt_tile<DT, BLK, NB>(a, blockIdx.x, tiles, bands, b0, part, red);
+    gemvt_tile<DT, BLK, NB>(a, blockIdx.x, tiles, bands, part, red);
   } else {
     outer_rows(a.dpre, oa, (int)blockIdx.x - gemvt_blocks, a.in, a.out);
+  }
+}
+
+// dX of 3 batch rows and more on the f64 matrix cores: the same exact terms
+// (f32 weight times f32 d_pre) in f64, every code row read once per 16 batch
+// rows. v_mfma_f64_16x16x4_f64 takes 16 batch rows x 4 code rows (A: lane l
+// holds d_pre of batch row l % 16, code row group l / 16) times 4 code rows x 16
+// columns. A lane decodes 16 consecutive columns of its group's code row, and
+// product j takes column j of every lane, so the 16 products of a step cover
+// 256 columns and no value moves between lanes. A workgroup owns 256 columns, 16
+// batch rows and a band of code rows in units of 16 (lane group g: rows 4 g ..
+// + 3 of a unit, one per step), its 8 waves consecutive runs of units. Their
+// sums are added in wave order through LDS, four batch rows at a time, into the
+// band's partial rows, or with a single band rounded into dX.
+// Bound by the matrix cores (64 cycles per product, 32 flops per cycle and SIMD,
+// as the f64 VALU, which here only decodes). 4096 x 4096 E4M3, whole backward
+// without dW: 3 rows 21.5 us, 32 rows 32, 64 rows 51 (0.56 us a row; 13.7 us of
+// products at 32 rows). k_bwd streamed the codes once per two batch rows: the
+// whole backward at 3 / 8 / 32 / 64 rows 48 / 98 / 353 / 694 us, now 38 / 45 / 97 /
+// 168; at 2 rows k_bwd takes 33.9.
+constexpr int kDxWaves = 8;
+constexpr int kDxCols = 256;
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+template <int DT, bool BLK>
+__global__ __launch_bounds__(64 * kDxWaves) void k_dx_mfma(GemvtArgs a, int batch, int tiles, int bands,
+                                                           int prows, double* __restrict__ part,
+                                                           float* __restrict__ dx) {
+  constexpr int kPitch = 17;  // doubles per lane: the 16 values of a lane, off the bank stride
+  __shared__ double red[kDxWaves][64 * kPitch];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, g = lane >> 4;
+  const int tile = blockIdx.x % tiles, band = blockIdx.x / tiles % bands, b0 = blockIdx.x / tiles / bands * 16;
+  const int col = tile * kDxCols + kCpl * c16;  // < kpad
+  const int units = (a.out + 15) / 16, runs = bands * kDxWaves, run = band * kDxWaves + wave;
+  const int u0 = (int)((int64_t)units * run / runs), u1 = (int)((int64_t)units * (run + 1) / runs);
+  typedef typename RowCodes<DT>::T Q;
+  const uint8_t* base = a.codes + (DT == kFP4 ? col / 2 : col);
+  const bool blive = b0 + c16 < batch;
+  const float* dp = a.dpre + (size_t)(blive ? b0 + c16 : 0) * a.out;
+  v4d acc[kCpl];
+#pragma unroll
+  for (int j = 0; j < kCpl; ++j) acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
+
+  struct Unit {
+    Q q[4];
+    float s[4], g[4];
+    uint8_t e[4];
+  };
+  auto load = [&](int u, Unit& p) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int o = 16 * u + 4 * g + s;  // < rpad
+      p.q[s] = *reinterpret_cast<const Q*>(base + (size_t)o * a.pitch);
+      if constexpr (BLK) p.e[s] = a.blk[(size_t)o * a.nblk + col / 32];
+      else p.s[s] = a.scale[o];
+      p.g[s] = dp[o < a.out ? o : a.out - 1];
+    }
+  };
+  auto add = [&](int u, const Unit& p) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      float w[kCpl];
+      decode16<DT>(p.q[s], w);
+      const float sf = BLK ? pow2f((int)p.e[s] - 127) : p.s[s];
+      const double gv = blive && 16 * u + 4 * g + s < a.out ? (double)p.g[s] : 0.0;
+#pragma unroll
+      for (int j = 0; j < kCpl; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(gv, (double)(w[j] * sf), acc[j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (u0 < u1) {
+    Unit p, q;
+    load(u0, p);
+    int u = u0;
+    for (; u + 2 <= u1; u += 2) {
+      load(u + 1, q);
+      __builtin_amdgcn_sched_barrier(0);
+      add(u, p);
+      load(u + 2 < u1 ? u + 2 : u + 1, p);
+      __builtin_amdgcn_sched_barrier(0);
+      add(u + 1, q);
+    }
+    if (u < u1) add(u, p);
+  }
+
+  // element i of D: batch row 4 i + g; column of product j: 16 c16 + j
+  const size_t cpad = (size_t)tiles * kDxCols;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kCpl; ++j) red[wave][lane * kPitch + j] = acc[j][i];
+    __syncthreads();
+    for (int t = threadIdx.x; t < 4 * kDxCols; t += 64 * kDxWaves) {
+      const int gg = t / kDxCols, c = t % kDxCols;
+      const int at = (16 * gg + c / kCpl) * kPitch + c % kCpl;
+      double v = red[0][at];
+#pragma unroll
+      for (int w = 1; w < kDxWaves; ++w) v += red[w][at];
+      const int b = b0 + 4 * i + gg, oc = tile * kDxCols + c;
+      if (bands > 1) {
+        part[((size_t)band * prows + b) * cpad + oc] = v;
+      } else if (b < batch && oc < a.in) {
+        dx[(size_t)b * a.in + oc] = (float)v;
+      }
+    }
+  }
+}
+
+// dW of more than 2 batch rows, as outer_rows with 8 rows per thread (the x
+// slice of a batch row is loaded and widened once for 8 rows) and the next
+// batch row's operands loaded ahead. Bound by the VALU: an element and batch row
+// takes an f64 FMA and the two conversions of its f32 rounding (3.4 operations
+// with the operands'): 4096 x 4096 1.78 us a row, 1.44 at the issue rate.
+constexpr int kOuterRowsB = 8;
+
+__global__ __launch_bounds__(kThreads) void k_outer(const float* __restrict__ dpre, OuterArgs oa, int in,
+                                                    int out) {
+  const int g = blockIdx.x, r0 = (g / oa.cb) * kOuterRowsB;
+  if (oa.dpre_out && g % oa.cb == 0) {  // as in outer_rows
+    for (int i = threadIdx.x; i < oa.batch * kOuterRowsB; i += kThreads) {
+      const int b = i / kOuterRowsB, r = r0 + i % kOuterRowsB;
+      if (r < out) oa.dpre_out[(size_t)b * out + r] = dpre[(size_t)b * out + r];
+    }
+  }
+  const int c = ((g % oa.cb) * kThreads + (int)threadIdx.x) * 4;
+  if (c >= in) return;
+  const ConstF32 dp = (ConstF32)dpre;
+  float acc[kOuterRowsB][4];
+#pragma unroll
+  for (int r = 0; r < kOuterRowsB; ++r)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[r][j] = 0.0f;
+  auto load = [&](int b, float (&xv)[4], float (&gr)[kOuterRowsB]) {
+    const float* xb = oa.x + (size_t)b * in + c;
+    if (oa.vec) {
+      const float4 t = *reinterpret_cast<const float4*>(xb);
+      xv[0] = t.x, xv[1] = t.y, xv[2] = t.z, xv[3] = t.w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xv[j] = c + j < in ? xb[j] : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < kOuterRowsB; ++r)
+      gr[r] = dp[(size_t)b * out + (r0 + r < out ? r0 + r : out - 1)];
+  };
+  float xn[4], gn[kOuterRowsB];
+  load(0, xn, gn);
+  for (int b = 0; b < oa.batch; ++b) {
+    double x[4], gr[kOuterRowsB];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = (double)xn[j];
+#pragma unroll
+    for (int r = 0; r < kOuterRowsB; ++r) gr[r] = (double)gn[r];
+    load(b + 1 < oa.batch ? b + 1 : b, xn, gn);
+#pragma unroll
+    for (int r = 0; r < kOuterRowsB; ++r)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[r][j] = (float)((double)acc[r][j] + gr[r] * x[j]);
+  }
+#pragma unroll
+  for (int r = 0; r < kOuterRowsB; ++r) {
+    if (r0 + r >= out) break;
+    float* dst = oa.dw + (size_t)(r0 + r) * in + c;
+    if (oa.vec) {
+      *reinterpret_cast<float4*>(dst) = make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (c + j < in) dst[j] = acc[r][j];
+    }
   }
 }
 
@@ -409,12 +585,36 @@ int gemvt_bands(int in, int out) {
   return bands < 1 ? 1 : bands;
 }
 
+// Column tiles, 16-row batch groups and code row bands of k_dx_mfma: one
+// workgroup per CU, and at least a unit of 16 code rows per wave.
+struct DxShape {
+  int tiles, groups, bands;
+};
+
+DxShape dx_shape(int in, int out, int batch) {
+  DxShape d;
+  d.tiles = (in + kDxCols - 1) / kDxCols;
+  d.groups = (batch + 15) / 16;
+  const int64_t wg = (int64_t)d.tiles * d.groups;
+  const int most = ((out + 15) / 16 + kDxWaves - 1) / kDxWaves;
+  int64_t bands = 256 / wg;
+  if (bands > most) bands = most;
+  d.bands = bands < 1 ? 1 : (int)bands;
+  return d;
+}
+
 template <int DT, bool BLK>
-void launch_bwd_t(const GemvtArgs& a, int b0, int nb, int tiles, int bands, int outer_blocks,
+void launch_dx_t(const GemvtArgs& a, const DxShape& d, int batch, double* part, float* dx, hipStream_t st) {
+  const unsigned grid = (unsigned)(d.tiles * d.bands * d.groups);
+  k_dx_mfma<DT, BLK><<<grid, 64 * kDxWaves, 0, st>>>(a, batch, d.tiles, d.bands, 16 * d.groups, part, dx);
+}
+
+template <int DT, bool BLK>
+void launch_bwd_t(const GemvtArgs& a, int nb, int tiles, int bands, int outer_blocks,
                   double* part, const OuterArgs& oa, hipStream_t st) {
   const unsigned grid = (unsigned)(tiles * bands + outer_blocks);
-  if (nb == 1) k_bwd<DT, BLK, 1><<<grid, kThreads, 0, st>>>(a, b0, tiles, bands, part, oa);
-  else k_bwd<DT, BLK, 2><<<grid, kThreads, 0, st>>>(a, b0, tiles, bands, part, oa);
+  if (nb == 1) k_bwd<DT, BLK, 1><<<grid, kThreads, 0, st>>>(a, tiles, bands, part, oa);
+  else k_bwd<DT, BLK, 2><<<grid, kThreads, 0, st>>>(a, tiles, bands, part, oa);
 }
 
 }  // namespace
@@ -430,9 +630,13 @@ Status launch_dpre(const float* g, const float* post, const float* pre, int act,
   return hip_status(hipGetLastError(), "dpre launch");
 }
 
-size_t gemvt_part_bytes(int in, int out) {
+size_t gemvt_part_bytes(int in, int out, int batch) {
+  if (batch > kStreamRows) {
+    const DxShape d = dx_shape(in, out, batch);
+    return d.bands > 1 ? (size_t)d.bands * d.groups * 16 * d.tiles * kDxCols * sizeof(double) : 16;
+  }
   const size_t cpad = (size_t)(in + kTileCols - 1) / kTileCols * kTileCols;
-  return (size_t)gemvt_bands(in, out) * kBatchChunk * cpad * sizeof(double);
+  return (size_t)gemvt_bands(in, out) * kStreamRows * cpad * sizeof(double);
 }
 
 Status launch_backward_products(const GemvtArgs& a, int dtype, bool blk, int batch,
@@ -454,22 +658,37 @@ Status launch_backward_products(const GemvtArgs& a, int dtype, bool blk, int bat
            (reinterpret_cast<uintptr_t>(dw) & 15u) == 0;
   const int64_t outer = (int64_t)(a.out + kOuterRows - 1) / kOuterRows * oa.cb;
   if (outer + (int64_t)tiles * bands >= (1ll << 31)) return Status::err(kUnsupported, "backward: too large");
-  for (int b0 = 0; b0 < batch; b0 += kBatchChunk) {
-    const int nb = batch - b0 < kBatchChunk ? batch - b0 : kBatchChunk;
-    // the dW workgroups ride with the first chunk (they cover every batch row)
-    const int ob = b0 == 0 ? (int)outer : 0;
+  if (batch > kStreamRows) {
+    const DxShape d = dx_shape(a.in, a.out, batch);
+    if ((int64_t)d.tiles * d.groups * d.bands >= (1ll << 27))  // 512 threads each
+      return Status::err(kUnsupported, "backward: too large");
     switch (dtype) {
-    case kE4M3: blk ? launch_bwd_t<kE4M3, true>(a, b0, nb, tiles, bands, ob, part, oa, st) : launch_bwd_t<kE4M3, false>(a, b0, nb, tiles, bands, ob, part, oa, st); break;
-    case kE5M2: blk ? launch_bwd_t<kE5M2, true>(a, b0, nb, tiles, bands, ob, part, oa, st) : launch_bwd_t<kE5M2, false>(a, b0, nb, tiles, bands, ob, part, oa, st); break;
-    case kFP4: blk ? launch_bwd_t<kFP4, true>(a, b0, nb, tiles, bands, ob, part, oa, st) : launch_bwd_t<kFP4, false>(a, b0, nb, tiles, bands, ob, part, oa, st); break;
+    case kE4M3: blk ? launch_dx_t<kE4M3, true>(a, d, batch, part, dx, st) : launch_dx_t<kE4M3, false>(a, d, batch, part, dx, st); break;
+    case kE5M2: blk ? launch_dx_t<kE5M2, true>(a, d, batch, part, dx, st) : launch_dx_t<kE5M2, false>(a, d, batch, part, dx, st); break;
+    case kFP4: blk ? launch_dx_t<kFP4, true>(a, d, batch, part, dx, st) : launch_dx_t<kFP4, false>(a, d, batch, part, dx, st); break;
     default: return Status::err(kUnsupported, "backward: dtype");
     }
     WV_HIP(hipGetLastError());
-    const dim3 rg((unsigned)((a.in + 63) / 64), (unsigned)nb);
-    k_gemvt_reduce<<<rg, kThreads, 0, st>>>(part, bands, nb, a.in, cpad, dx + (size_t)b0 * a.in);
-    WV_HIP(hipGetLastError());
+    if (d.bands > 1) {
+      const dim3 rg((unsigned)((a.in + 63) / 64), (unsigned)batch);
+      k_gemvt_reduce<<<rg, kThreads, 0, st>>>(part, d.bands, 16 * d.groups, a.in, (size_t)d.tiles * kDxCols, dx);
+      WV_HIP(hipGetLastError());
+    }
+    const int64_t wgs = (int64_t)(a.out + kOuterRowsB - 1) / kOuterRowsB * oa.cb;
+    k_outer<<<(unsigned)wgs, kThreads, 0, st>>>(a.dpre, oa, a.in, a.out);
+    return hip_status(hipGetLastError(), "outer launch");
   }
-  return Status::ok();
+  const int ob = (int)outer;
+  switch (dtype) {
+  case kE4M3: blk ? launch_bwd_t<kE4M3, true>(a, batch, tiles, bands, ob, part, oa, st) : launch_bwd_t<kE4M3, false>(a, batch, tiles, bands, ob, part, oa, st); break;
+  case kE5M2: blk ? launch_bwd_t<kE5M2, true>(a, batch, tiles, bands, ob, part, oa, st) : launch_bwd_t<kE5M2, false>(a, batch, tiles, bands, ob, part, oa, st); break;
+  case kFP4: blk ? launch_bwd_t<kFP4, true>(a, batch, tiles, bands, ob, part, oa, st) : launch_bwd_t<kFP4, false>(a, batch, tiles, bands, ob, part, oa, st); break;
+  default: return Status::err(kUnsupported, "backward: dtype");
+  }
+  WV_HIP(hipGetLastError());
+  const dim3 rg((unsigned)((a.in + 63) / 64), (unsigned)batch);
+  k_gemvt_reduce<<<rg, kThreads, 0, st>>>(part, bands, batch, a.in, cpad, dx);
+  return hip_status(hipGetLastError(), "backward reduce launch");
 }
 
 Status launch_swiglu_bwd(const float* gate_pre, const float* up_post, const float* grad_h,

@@ -302,7 +302,7 @@ struct GemvtArgs {
   const float* dpre = nullptr;     // [batch][out]
 };
 // Bytes of the f64 partial buffer launch_backward_products needs.
-size_t gemvt_part_bytes(int in, int out);
+size_t gemvt_part_bytes(int in, int out, int batch);
 // dX [batch][in] = W^T d_pre (f64 accumulation, rounded once to f32) and dW
 // [out][in] (the reference's per-batch-row f32 accumulation) from d_pre.
 // With dpre_out set, a.dpre is gy of a Linear layer without a target (d_pre

@@ -489,7 +489,7 @@ Status dense_backward(const DenseLayer& L, int batch, const float* x, const floa
   if (!direct)
     WV_TRY(launch_dpre(g, post, pre, linear_act ? kLinear : L.act, use_target ? 1 : 0, n, dpre,
                        loss_part, st));
-  const size_t pb = gemvt_part_bytes(L.in, L.out);
+  const size_t pb = gemvt_part_bytes(L.in, L.out, batch);
   if (ws->d.bytes < pb) WV_TRY(ws->d.alloc(pb));
   GemvtArgs a;
   a.codes = L.dev.d_codes();
