@@ -56,14 +56,15 @@ __global__ void k_rope_table(double* __restrict__ tab, int tokens, int hd, doubl
 // (num_kv) rows of token t by angle t / theta^(2d/hd), in f64 (cos and sin
 // from the table when one is given).
 __global__ void k_rope(float* __restrict__ q, float* __restrict__ k, int tokens, int heads,
-                       int kv_heads, int hd, double theta, const double* __restrict__ tab) {
+                       int kv_heads, int hd, int q_stride, int kv_stride, double theta,
+                       const double* __restrict__ tab) {
   const int t = blockIdx.x;
   const int half = hd / 2;
   const int per_tok = (heads + kv_heads) * half;
   for (int i = threadIdx.x; i < per_tok; i += blockDim.x) {
     const int h = i / half, d = i % half;
-    float* row = h < heads ? q + ((size_t)t * heads + h) * hd
-                           : k + ((size_t)t * kv_heads + (h - heads)) * hd;
+    float* row = h < heads ? q + (size_t)t * q_stride + (size_t)h * hd
+                           : k + (size_t)t * kv_stride + (size_t)(h - heads) * hd;
     double c, s;
     if (tab) {
       c = tab[2 * (t * half + d)];
@@ -90,7 +91,7 @@ __device__ __forceinline__ void attend_token(const AttnArgs& a, int t, int h, in
   const int kv_len = b * a.seq + a.seq;
   const int last = kv_len - 1;
   const int kvh = h / (a.heads / a.kv_heads);
-  const int kvd = a.kv_heads * a.hd;
+  const int kvd = a.kv_stride;
 
   float m = -INFINITY, l = 0.0f;
 #pragma unroll
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
   const int lane = threadIdx.x;
   const size_t row = (size_t)t * a.heads * a.hd + (size_t)h * a.hd;
   __shared__ float qs[256];
-  for (int d = lane; d < a.hd; d += 64) qs[d] = a.q[row + d];
+  for (int d = lane; d < a.hd; d += 64) qs[d] = a.q[(size_t)t * a.q_stride + (size_t)h * a.hd + d];
   __syncthreads();
   float acc[kMaxHdPerLane];
   attend_token(a, t, h, lane, qs, acc);
@@ -342,7 +343,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
   const int b = blockIdx.x / qblocks, qb = blockIdx.x % qblocks;
   const int h = blockIdx.y;
   const int kvh = h / (a.heads / a.kv_heads);
-  const int qd = a.heads * HD, kvd = a.kv_heads * HD;
+  const int qd = a.heads * HD, kvd = a.kv_stride;
   const int last = b * a.seq + a.seq - 1;
   const int p_lo = last - a.msl + 1 > 0 ? last - a.msl + 1 : 0;
   const int s_q = qb * kQB + wave * 16 + c16;      // query within the sequence
@@ -372,7 +373,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
   // TT bf16 terms (each the rounded remainder of those before it)
   bf16x8 qop[KS][TT];
   {
-    const float* qrow = a.q + (size_t)qp * qd + (size_t)h * HD;
+    const float* qrow = a.q + (size_t)qp * a.q_stride + (size_t)h * HD;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const v4f q0 = *reinterpret_cast<const v4f*>(qrow + 32 * ks + 8 * g);
@@ -688,7 +689,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       const int t = b * a.seq + sj;
       const size_t row = (size_t)t * qd + (size_t)h * HD;
       float acc[kMaxHdPerLane];
-      attend_token(a, t, h, lane, a.q + row, acc);
+      attend_token(a, t, h, lane, a.q + (size_t)t * a.q_stride + (size_t)h * HD, acc);
 #pragma unroll
       for (int i = 0; i < (HD + 63) / 64; ++i) {
         const int d = lane + 64 * i;
@@ -792,13 +793,17 @@ static void attn_hd(const AttnArgs& a, hipStream_t st) {
 Status launch_attention(const AttnArgs& a, hipStream_t st) {
   if (a.hd > 64 * kMaxHdPerLane || a.hd % 4 != 0)
     return Status::err(kUnsupported, "attention: head_dim must be a multiple of 4 and <= 256");
+  if (a.q_stride < a.heads * a.hd || a.kv_stride < a.kv_heads * a.hd ||
+      ((a.q_stride | a.kv_stride) & 3) != 0)
+    return Status::err(kInvalid, "attention: token strides");
   const bool fast = attention_fast(a);
   if (a.split && (!attention_writes_split(a) || a.split_mpad < a.tokens || a.split_mpad % 16 != 0))
     return Status::err(kInvalid, "attention: the output split needs the matrix-core path, "
                                  "heads * hd % 256 == 0 and seq % 16 == 0");
   if (a.rope) {
     k_rope<<<a.tokens, 256, 0, st>>>(const_cast<float*>(a.q), const_cast<float*>(a.k), a.tokens,
-                                     a.heads, a.kv_heads, a.hd, a.rope_theta, a.rope_tab);
+                                     a.heads, a.kv_heads, a.hd, a.q_stride, a.kv_stride,
+                                     a.rope_theta, a.rope_tab);
     WV_HIP(hipGetLastError());
   }
   if (fast) {

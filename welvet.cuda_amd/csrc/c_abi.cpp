@@ -689,6 +689,7 @@ welvet_status welvet_mha_mount(int32_t batch, int32_t seq, int32_t d_model, int3
     if (st && terms != wv::kTerms)
       st = Status::err(wv::kUnsupported, "mha: two activation terms are for Dense layers");
     if (st) st = wv::mha_build(cfg, dtype, scheme, Q, K, V, O, &s->layer, s->stream.s);
+    if (st) st = wv::mha_prepare_rows(&s->layer, batch * seq, s->stream.s);
     if (st) st = wv::mha_prepare(s->layer, batch, seq, &s->ws);
     if (st) st = s->x.alloc(T * d_model * sizeof(float));
     if (st) st = s->pre.alloc(T * cfg.q_dim() * sizeof(float));

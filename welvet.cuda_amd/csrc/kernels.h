@@ -209,8 +209,9 @@ struct MxgArgs {
   // applies RoPE to the output (row m = token position m, heads of rope_hd
   // columns, 128 % rope_hd == 0): pairs (d, d + rope_hd/2) rotated by the
   // (cos, sin) table [token][pair] in f64, as build_rope_table makes it
+  // Columns from rope_n on are left as they are (a multiple of rope_hd)
   const double* rope_tab = nullptr;
-  int rope_hd = 0;
+  int rope_hd = 0, rope_n = 0;
   // large tiles, one matrix, N a multiple of 256: when set, the epilogue also
   // writes the split of post here, laid out as the split buffer of a layer
   // with the same rows (mpad) and kpad = N (the next layer of a chain, which
@@ -264,6 +265,9 @@ struct AttnArgs {
   const float* q = nullptr;  // [tokens][heads*hd], rotated in place when rope
   const float* k = nullptr;  // [tokens][kv_heads*hd], rotated in place when rope
   const float* v = nullptr;  // [tokens][kv_heads*hd]
+  // floats from a token's row to the next one's, in q and in k and v
+  // (multiples of 4)
+  int q_stride = 0, kv_stride = 0;
   float* out = nullptr;      // [tokens][heads*hd]
   int tokens = 0, seq = 0, heads = 0, kv_heads = 0, hd = 0, msl = 0;
   int mask = 1, window = 0, prefix_len = 0, window_causal = 1;

@@ -421,7 +421,7 @@ static Status fix_nonfinite(const DenseLayer& L, int batch, const float* x, int 
 Status dense_forward_split(const DenseLayer& L, int batch, const float* x, bool split_ready,
                            Workspace* ws, float* pre, float* post, hipStream_t st,
                            const double* rope_tab, int rope_hd, bool keep_out,
-                           uint8_t* next_split) {
+                           uint8_t* next_split, int rope_n) {
   MxgArgs p = mxg_args(L, batch, split_buf(ws));
   p.pre = pre;
   p.post = post;
@@ -429,6 +429,7 @@ Status dense_forward_split(const DenseLayer& L, int batch, const float* x, bool 
   p.keep_out = keep_out ? 1 : 0;
   p.rope_tab = rope_tab;
   p.rope_hd = rope_hd;
+  p.rope_n = rope_n ? rope_n : L.out;
   if (mxg_block_m(batch) > 16) {
     if (!split_ready)
       WV_TRY(launch_split(x, L.in, batch, L.in, L.dev.kpad, split_buf(ws), st, L.terms));
@@ -944,7 +945,72 @@ Status mha_build(const MHAConfig& cfg_in, int dtype, int scheme, const float* Q,
   WV_TRY(dense_build(d, kvd, kLinear, dtype, scheme, K, nullptr, 0, &L->k, st));
   WV_TRY(dense_build(d, kvd, kLinear, dtype, scheme, V, nullptr, 0, &L->v, st));
   WV_TRY(dense_build(qd, d, kLinear, dtype, scheme, O, nullptr, 0, &L->o, st));
+  return mha_join(L, st);
+}
+
+// Q, K and V read the same rows of x. One product of qd + 2 kvd outputs in
+// the place of three takes two launches less (four at 5-32 tokens, whose
+// product is followed by a reduction over its K ranges), and its workgroups
+// fill the GPU where each of the three leaves most of it idle (100 tokens of 12
+// heads over 4 K/V heads of 64: 6, 2 and 2 of the 256 CUs). Whole layers of 12
+// heads over 4 of 64, us with three products and with one: 1 token 20.2 / 13.6,
+// 24 tokens 45.4 / 25.8, 100 tokens 55.1 / 26.9, 500 tokens 79.3 / 48.6; 4 x 512
+// tokens of 16 heads over 4 121 / 81. The copy replaces the three matrices.
+Status mha_join(MHALayer* L, hipStream_t st) {
+  DenseLayer* parts[3] = {&L->q, &L->k, &L->v};
+  const DeviceWeights& d0 = L->q.dev;
+  int rows = 0;
+  for (const DenseLayer* p : parts) {
+    const DeviceWeights& d = p->dev;
+    // row blocks of 16 stay whole (blk_frag), and the attention kernels read
+    // 16-byte vectors of the joined rows
+    if (p->format || p->need_epi() || d.nf_count() != 0 || !d.codes.p || d.dtype != d0.dtype ||
+        d.scheme != d0.scheme || d.kpad != d0.kpad || p->in != L->q.in ||
+        p->terms != L->q.terms || p->out % 16 != 0)
+      return Status::ok();
+    rows += p->out;
+  }
+  DenseLayer& J = L->qkv;
+  DeviceWeights& j = J.dev;
+  J.in = L->q.in, J.act = kLinear, J.terms = L->q.terms;
+  j.dtype = d0.dtype, j.scheme = d0.scheme, j.rows = rows, j.cols = d0.cols;
+  j.rpad = (int)round_up(rows, kRowPad), j.kpad = d0.kpad, j.pitch = d0.pitch, j.nblk = d0.nblk;
+  // a row's bytes in each array, and the 32-bit value its padding rows hold
+  const bool blk = j.scheme == kSchemeBlock32;
+  struct Array {
+    DevBuf DeviceWeights::*buf;
+    size_t row;
+    int pad;
+  } const arrays[4] = {
+      {&DeviceWeights::codes, (size_t)j.pitch, 0},
+      {&DeviceWeights::row_scale, sizeof(float), 0x3f800000},  // 1.0f
+      {&DeviceWeights::blk, blk ? (size_t)j.nblk : 0, 0x7f7f7f7f},
+      {&DeviceWeights::blk_frag, blk ? (size_t)(j.kpad + 511) / 512 * 16 : 0, 0x7f7f7f7f},
+  };
+  for (const Array& a : arrays) {
+    if (!a.row) continue;
+    DevBuf& dst = j.*a.buf;
+    WV_TRY(dst.alloc((size_t)j.rpad * a.row));
+    WV_HIP(hipMemsetD32Async(dst.p, a.pad, dst.bytes / 4, st));
+    size_t at = 0;
+    for (const DenseLayer* p : parts) {
+      const DevBuf& src = p->dev.*a.buf;
+      const size_t n = (size_t)p->out * a.row;
+      if (src.bytes < n) return Status::err(kInternal, "mha: joined array shorter than its rows");
+      WV_HIP(hipMemcpyAsync(dst.as<char>() + at, src.p, n, hipMemcpyDeviceToDevice, st));
+      at += n;
+    }
+  }
+  WV_TRY(hip_status(hipStreamSynchronize(st), "mha join"));
+  for (DenseLayer* p : parts)
+    for (const Array& a : arrays) (p->dev.*a.buf).reset();
+  J.out = rows;
   return Status::ok();
+}
+
+Status mha_prepare_rows(MHALayer* L, int tokens, hipStream_t st) {
+  if (L->qkv.out) WV_TRY(dense_prepare_rows(&L->qkv, tokens, st));
+  return dense_prepare_rows(&L->o, tokens, st);
 }
 
 size_t mha_workspace_bytes(const MHALayer& L, int batch, int seq) {
@@ -955,7 +1021,8 @@ size_t mha_workspace_bytes(const MHALayer& L, int batch, int seq) {
 static size_t mha_split_bytes(const MHALayer& L, int T) {
   if (!uses_split(T)) return 0;
   size_t n = 0;
-  for (const DenseLayer* d : {&L.q, &L.k, &L.v, &L.o}) {
+  for (const DenseLayer* d : {&L.q, &L.k, &L.v, &L.o, &L.qkv}) {
+    if (d->out == 0) continue;
     const size_t b = gemm_ws_bytes(*d, T, 1);
     n = b > n ? b : n;
   }
@@ -998,8 +1065,10 @@ Status mha_forward(const MHALayer& L, int batch, int seq, const float* x, float*
   if (ws->a.bytes < need) WV_TRY(ws->a.alloc(need));
   const int T = batch * seq;
   float* qb = ws->a.as<float>();
-  float* kb = qb + (size_t)T * c.q_dim();
-  float* vb = kb + (size_t)T * c.kv_dim();
+  // joined: a token's Q, K and V follow each other in one row
+  const bool joined = L.qkv.out != 0;
+  float* kb = qb + (joined ? 1 : (size_t)T) * c.q_dim();
+  float* vb = kb + (joined ? 1 : (size_t)T) * c.kv_dim();
   // RoPE in the Q and K GEMM epilogues (large tiles): the attention kernel
   // then reads rotated rows
   const bool rope = mha_rope(c);
@@ -1007,9 +1076,20 @@ Status mha_forward(const MHALayer& L, int batch, int seq, const float* x, float*
   // rotation pairs each column with another)
   const bool rope_epi = rope && uses_split(T) && mxg_block_m(T) > 16 && c.head_dim % 8 == 0 &&
                         128 % c.head_dim == 0 && !L.q.need_epi() && !L.k.need_epi() &&
-                        L.q.dev.nf_count() == 0 && L.k.dev.nf_count() == 0;
+                        L.q.dev.nf_count() == 0 && L.k.dev.nf_count() == 0 &&
+                        // a joined product of few tiles is split along K and
+                        // followed by k_rope
+                        !(joined && mxg_part_bytes(T, L.qkv.dev.kpad, L.qkv.out, 1) > 0);
   if (rope) WV_TRY(ensure_rope_table(L, T, ws, st));
-  if (uses_split(T)) {
+  if (joined && uses_split(T)) {
+    WV_TRY(ensure_split(ws, mha_split_bytes(L, T)));
+    // (read by the attention kernel next: kept in the caches)
+    WV_TRY(dense_forward_split(L.qkv, T, x, false, ws, qb, nullptr, st,
+                               rope_epi ? ws->c.as<const double>() : nullptr,
+                               rope_epi ? c.head_dim : 0, true, nullptr, c.q_dim() + c.kv_dim()));
+  } else if (joined) {
+    WV_TRY(dense_forward(L.qkv, T, x, qb, nullptr, ws, st));
+  } else if (uses_split(T)) {
     // Q, K and V read the same activations: above 32 rows they are split
     // once (up to 32 rows each GEMM kernel splits its own K range)
     WV_TRY(ensure_split(ws, mha_split_bytes(L, T)));
@@ -1029,6 +1109,8 @@ Status mha_forward(const MHALayer& L, int batch, int seq, const float* x, float*
   }
   AttnArgs a;
   a.q = qb, a.k = kb, a.v = vb, a.out = attn;
+  a.q_stride = joined ? L.qkv.out : c.q_dim();
+  a.kv_stride = joined ? L.qkv.out : c.kv_dim();
   a.tokens = T, a.seq = seq, a.heads = c.num_heads, a.kv_heads = c.num_kv_heads;
   a.hd = c.head_dim, a.msl = c.max_seq_len;
   a.mask = c.mask, a.window = c.window, a.prefix_len = c.prefix_len;

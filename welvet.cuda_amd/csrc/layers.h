@@ -160,13 +160,14 @@ inline uint8_t* split_buf(Workspace* ws) { return ws->b.as<uint8_t>(); }
 // reads the split terms of x from split_buf(ws), made here unless
 // `split_ready` (launch_split of x with L.dev.kpad already ran); up to 32
 // rows the GEMM kernel splits x itself. keep_out: the next launch reads the
-// output (MxgArgs::keep_out).
+// output (MxgArgs::keep_out). rope_n: the columns that RoPE turns (0: all).
 // next_split: the reduce of this layer's K-split product also writes the
 // split of post there, for `next` (dense_fuses_next must hold).
 Status dense_forward_split(const DenseLayer& L, int batch, const float* x, bool split_ready,
                            Workspace* ws, float* pre, float* post, hipStream_t st,
                            const double* rope_tab = nullptr, int rope_hd = 0,
-                           bool keep_out = false, uint8_t* next_split = nullptr);
+                           bool keep_out = false, uint8_t* next_split = nullptr,
+                           int rope_n = 0);
 // True when `batch` rows of L and then `next` (whose input is L's post) can
 // run with L's K-split reduce writing next's split terms: both on the
 // split matrix-core path above 32 rows, L's product split along K, N a
@@ -257,7 +258,16 @@ Status mha_validate(MHAConfig* c);
 struct MHALayer {
   MHAConfig cfg;
   DenseLayer q, k, v, o;
+  // Q, K and V rows one after the other (mha_join); out is 0 without it. The
+  // three layers then keep their stores and shapes, and no device weights.
+  DenseLayer qkv;
 };
+// Joins the built Q, K and V matrices into one, so that a forward runs one
+// product for the three. Left as they are where their storage, biases or rows
+// with non-finite codes keep them apart.
+Status mha_join(MHALayer* L, hipStream_t st);
+// dense_prepare_rows for the matrices of a forward of `tokens` tokens.
+Status mha_prepare_rows(MHALayer* L, int tokens, hipStream_t st);
 Status mha_build(const MHAConfig& cfg, int dtype, int scheme, const float* Q, const float* K,
                  const float* V, const float* O, MHALayer* L, hipStream_t st);
 // x [batch*seq][d] -> attn [batch*seq][q_dim] (pre), y [batch*seq][d] (post).

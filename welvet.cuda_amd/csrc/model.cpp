@@ -372,6 +372,7 @@ void build(ModelNode& c, int scheme, int terms, hipStream_t st) {
                             s.bias.size(), parts[i], st));
       parts[i]->terms = terms;
     }
+    good(mha_join(c.mha.get(), st));
     break;
   }
   case 19:

@@ -227,6 +227,7 @@ __device__ __forceinline__ MxgArgs load_args(ConstArgs t) {
   p.next = t->next;
   p.rope_tab = t->rope_tab;
   p.rope_hd = t->rope_hd;
+  p.rope_n = t->rope_n;
   p.terms = t->terms;
   p.keep_out = t->keep_out;
   return p;
@@ -678,7 +679,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4, W
         const int r = rr * RPI + lane / LPR;
         float4 y = *reinterpret_cast<const float4*>(&stage[wave][r][cl]);
         if constexpr (MATS == 1 && CH == 128) {
-          if (p.rope_tab) {
+          if (p.rope_tab && n < p.rope_n) {
             // the 4 columns sit in one half of one head; the partner columns
             // are in the same staged chunk (128 % rope_hd == 0)
             const int half = p.rope_hd >> 1;
@@ -1587,7 +1588,7 @@ int mxg_ksplit(int M, int kpad, int N, int mats) {
 template <int DT, bool BLK, int MATS>
 Status launch_t(const MxgArgs& p, int bm, hipStream_t st) {
   if (p.rope_tab && (bm != kBM || MATS != 1 || p.need_epi || p.next || p.rope_hd <= 0 ||
-                     p.rope_hd % 8 != 0 || 128 % p.rope_hd != 0))
+                     p.rope_hd % 8 != 0 || 128 % p.rope_hd != 0 || p.rope_n % p.rope_hd != 0))
     return Status::err(kInvalid, "mxg: RoPE epilogue needs the large tiles, one matrix, no epilogue");
   if (bm == kBM) {
     if ((size_t)kTerms * p.mpad * p.kpad >= (1ull << 31) ||
