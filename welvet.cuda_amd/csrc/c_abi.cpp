@@ -256,13 +256,10 @@ welvet_status welvet_dense_execute(welvet_dense_session* s, const float* x, floa
     const size_t xb = (size_t)s->batch * s->layer.in * sizeof(float);
     const size_t yb = (size_t)s->batch * s->layer.out * sizeof(float);
     hipStream_t st = s->stream.s;
-    WV_TRY(wv::copy_h2d(s->x.p, x, xb, st));
-    WV_TRY(wv::dense_forward(s->layer, s->batch, s->x.as<float>(), s->pre.as<float>(),
-                             s->post.as<float>(), &s->ws, st));
-    WV_TRY(wv::copy_d2h(pre, s->pre.p, yb, st));
-    WV_TRY(wv::copy_d2h(post, s->post.p, yb, st));
-    WV_HIP(hipStreamSynchronize(st));
-    return Status::ok();
+    return wv::host_call(x, s->x.p, xb, pre, s->pre.p, yb, post, s->post.p, yb, st, [&] {
+      return wv::dense_forward(s->layer, s->batch, s->x.as<float>(), s->pre.as<float>(),
+                               s->post.as<float>(), &s->ws, st);
+    });
   });
 }
 
@@ -621,13 +618,10 @@ welvet_status welvet_swiglu_execute(welvet_swiglu_session* s, const float* x, fl
     const size_t xb = (size_t)s->rows * s->layer.in * sizeof(float);
     const size_t hb = (size_t)s->rows * s->layer.inter * sizeof(float);
     hipStream_t st = s->stream.s;
-    WV_TRY(wv::copy_h2d(s->x.p, x, xb, st));
-    WV_TRY(wv::swiglu_forward(s->layer, s->rows, s->x.as<float>(), s->pre.as<float>(),
-                              s->post.as<float>(), &s->ws, st));
-    WV_TRY(wv::copy_d2h(pre, s->pre.p, hb, st));
-    WV_TRY(wv::copy_d2h(post, s->post.p, xb, st));
-    WV_HIP(hipStreamSynchronize(st));
-    return Status::ok();
+    return wv::host_call(x, s->x.p, xb, pre, s->pre.p, hb, post, s->post.p, xb, st, [&] {
+      return wv::swiglu_forward(s->layer, s->rows, s->x.as<float>(), s->pre.as<float>(),
+                                s->post.as<float>(), &s->ws, st);
+    });
   });
 }
 
@@ -712,13 +706,10 @@ welvet_status welvet_mha_execute(welvet_mha_session* s, const float* x, float* p
     const size_t xb = T * s->layer.cfg.d_model * sizeof(float);
     const size_t ab = T * s->layer.cfg.q_dim() * sizeof(float);
     hipStream_t st = s->stream.s;
-    WV_TRY(wv::copy_h2d(s->x.p, x, xb, st));
-    WV_TRY(wv::mha_forward(s->layer, s->batch, s->seq, s->x.as<float>(), s->pre.as<float>(),
-                           s->post.as<float>(), &s->ws, st));
-    WV_TRY(wv::copy_d2h(pre, s->pre.p, ab, st));
-    WV_TRY(wv::copy_d2h(post, s->post.p, xb, st));
-    WV_HIP(hipStreamSynchronize(st));
-    return Status::ok();
+    return wv::host_call(x, s->x.p, xb, pre, s->pre.p, ab, post, s->post.p, xb, st, [&] {
+      return wv::mha_forward(s->layer, s->batch, s->seq, s->x.as<float>(), s->pre.as<float>(),
+                             s->post.as<float>(), &s->ws, st);
+    });
   });
 }
 

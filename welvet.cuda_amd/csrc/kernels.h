@@ -291,6 +291,16 @@ bool attention_writes_split(const AttnArgs& a);
 // in f64: tab[2 * (t * (hd/2) + d) + {0, 1}].
 Status build_rope_table(double* tab, int tokens, int hd, double theta, hipStream_t st);
 
+// ---- copies by a kernel (hostio.hip) ----
+// Device memory or pinned host memory on either side; 16-byte aligned, whole
+// 4-byte words.
+struct CopyRange {
+  void* dst = nullptr;
+  const void* src = nullptr;
+  size_t bytes = 0;
+};
+Status launch_copy(const CopyRange& a, const CopyRange& b, hipStream_t st);
+
 // ---- Dense backward and SGD (backward.hip) ----
 // d_pre = f32(f64(gy) * act'(f64 pre)) over n = batch * out elements; with
 // use_target, g holds the target and gy = f32(2/n (post - target)), and

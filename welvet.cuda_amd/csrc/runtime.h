@@ -1,6 +1,7 @@
 // Device runtime (device 0, identity) and an owning stream handle.
 #pragma once
 
+#include <functional>
 #include <string>
 
 #include "common.h"
@@ -22,6 +23,13 @@ int cu_count();
 // before it is complete). Calls from different threads serialize.
 Status copy_h2d(void* dst, const void* src, size_t n, hipStream_t st);
 Status copy_d2h(void* dst, const void* src, size_t n, hipStream_t st);
+
+// One forward call on host buffers: x (xb bytes) to dx, `run` queued on `st`,
+// then pre and post (yb and zb bytes) from dpre and dpost; complete on return.
+// Device buffers are 16-byte aligned and sizes are whole floats.
+Status host_call(const void* x, void* dx, size_t xb, void* pre, const void* dpre, size_t yb,
+                 void* post, const void* dpost, size_t zb, hipStream_t st,
+                 const std::function<Status()>& run);
 
 // Owning HIP stream at the default priority.
 struct Stream {
