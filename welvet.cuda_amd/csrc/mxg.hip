@@ -96,9 +96,9 @@ __global__ __launch_bounds__(kThreads) void k_split(const float* __restrict__ x,
 
   __shared__ __attribute__((aligned(16))) float stage[kWaves][16][132];
   float(*sl)[132] = stage[wave];  // rows padded by 16 bytes: no bank conflicts below
-  // Unconditional loads clamped to the last row and column (16-byte loads
-  // when VEC: x aligned, cols and x_stride multiples of 4), then zeroed
-  // outside [0, M) x [0, cols).
+  // Unconditional 16-byte loads clamped to the last row and column, then
+  // zeroed outside [0, M) x [0, cols). VEC: x aligned, cols and x_stride
+  // multiples of 4; load4_any otherwise.
   const GlobalF xg = (GlobalF)x;
   const int c4 = 4 * (lane & 31), k = kc * 128 + c4;
   float4 xv[8];
@@ -110,10 +110,7 @@ __global__ __launch_bounds__(kThreads) void k_split(const float* __restrict__ x,
       const f32x4 t = *reinterpret_cast<const __attribute__((address_space(1))) f32x4*>(row + (k < cols ? k : 0));
       xv[i] = make_float4(t.x, t.y, t.z, t.w);
     } else {
-      xv[i].x = row[k < cols ? k : cols - 1];
-      xv[i].y = row[k + 1 < cols ? k + 1 : cols - 1];
-      xv[i].z = row[k + 2 < cols ? k + 2 : cols - 1];
-      xv[i].w = row[k + 3 < cols ? k + 3 : cols - 1];
+      xv[i] = load4_any(row, k, cols);
     }
   }
 #pragma unroll
@@ -828,7 +825,7 @@ int mxs_ksplit(int N, int kpad, int mpad) {
   return ks < S ? ks : S;
 }
 
-template <int DT, bool BLK, int MATS, int MB, int RB, int KRT, int D, bool XV, int NT>
+template <int DT, bool BLK, int MATS, int MB, int RB, int KRT, int D, int NT>
 __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mxs(
     MxgArgs p, int ksplit) {
   constexpr int ROWS = 16 * kSmallWaves * RB;  // weight rows per workgroup
@@ -898,8 +895,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_e
   // chunk r), j = b * KR + r, goes to wave j % 8. Each lane loads the 32
   // values of its operand (row b * 16 + i16, k = 64h + 16g + .. for E4M3
   // terms, k = 32g + .. for FP6 terms), with
-  // unconditional loads clamped to the last unit, row and column (16-byte
-  // loads when XV: x aligned, cols and stride multiples of 4). The first
+  // unconditional 16-byte loads clamped to the last unit, row and column. The first
   // unit's loads are issued before the first D - 1 chunks of weights, so its
   // split waits for them only and the weights stay in flight under it; a
   // wave's further units (K ranges above 8 chunks) load after it.
@@ -911,7 +907,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_e
     const int row = (j / KR) * 16 + i16;
     const float* src = p.x + (size_t)(row < p.M ? row : p.M - 1) * p.x_stride;
     const int kb = (k0 + j % KR) * 128 + (X6 ? 32 : 16) * g;
-    if constexpr (XV) {
+    if (p.x_vec) {  // uniform
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int k = X6 ? kb + 4 * q : kb + 64 * (q >> 2) + 4 * (q & 3);
@@ -921,10 +917,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int k = X6 ? kb + 4 * q : kb + 64 * (q >> 2) + 4 * (q & 3);
-        xin[q].x = src[k < p.cols ? k : p.cols - 1];
-        xin[q].y = src[k + 1 < p.cols ? k + 1 : p.cols - 1];
-        xin[q].z = src[k + 2 < p.cols ? k + 2 : p.cols - 1];
-        xin[q].w = src[k + 3 < p.cols ? k + 3 : p.cols - 1];
+        xin[q] = load4_any((GlobalF)src, k, p.cols);
       }
     }
   };
@@ -1519,7 +1512,7 @@ Status launch_rows(const MxgArgs& p, hipStream_t st) {
   return hip_status(hipGetLastError(), "mxr launch");
 }
 
-template <int DT, bool BLK, int MATS, int MB, int RB, int KRT, bool XV = true>
+template <int DT, bool BLK, int MATS, int MB, int RB, int KRT>
 void launch_small_krt(const MxgArgs& p, int ksplit, hipStream_t st) {
   constexpr int NT3 = kTerms;
   // ring depth: 6-14 KiB of weights in flight per wave within the register
@@ -1532,20 +1525,18 @@ void launch_small_krt(const MxgArgs& p, int ksplit, hipStream_t st) {
   // two activation terms: Dense only (one matrix)
   if constexpr (MATS == 1) {
     if (p.terms == 2) {
-      k_mxs<DT, BLK, MATS, MB, RB, KRT, D, XV, 2><<<grid, 64 * kSmallWaves, 0, st>>>(p, ksplit);
+      k_mxs<DT, BLK, MATS, MB, RB, KRT, D, 2><<<grid, 64 * kSmallWaves, 0, st>>>(p, ksplit);
       return;
     }
   }
-  k_mxs<DT, BLK, MATS, MB, RB, KRT, D, XV, NT3><<<grid, 64 * kSmallWaves, 0, st>>>(p, ksplit);
+  k_mxs<DT, BLK, MATS, MB, RB, KRT, D, NT3><<<grid, 64 * kSmallWaves, 0, st>>>(p, ksplit);
 }
 
 template <int DT, bool BLK, int MATS, int MB, int RB>
 void launch_small_rb(const MxgArgs& p, int ksplit, hipStream_t st) {
   const int S = p.kpad / 128, kr = (S + ksplit - 1) / ksplit;  // largest range
   constexpr int K1 = MB == 1 ? 4 : 4, K2 = MB == 1 ? 8 : 8, K3 = MB == 1 ? 12 : 12;
-  // element loads of an unaligned input: one variant (the largest range)
-  if (!p.x_vec) launch_small_krt<DT, BLK, MATS, MB, RB, small_krt_max(MB), false>(p, ksplit, st);
-  else if (kr <= K1) launch_small_krt<DT, BLK, MATS, MB, RB, K1>(p, ksplit, st);
+  if (kr <= K1) launch_small_krt<DT, BLK, MATS, MB, RB, K1>(p, ksplit, st);
   else if (kr <= K2) launch_small_krt<DT, BLK, MATS, MB, RB, K2>(p, ksplit, st);
   else if (kr <= K3 || MB == 2) launch_small_krt<DT, BLK, MATS, MB, RB, K3>(p, ksplit, st);
   else if (kr <= 16) launch_small_krt<DT, BLK, MATS, MB, RB, (MB == 1 ? 16 : 12)>(p, ksplit, st);

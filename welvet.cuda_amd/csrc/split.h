@@ -29,6 +29,20 @@ typedef short v2s __attribute__((ext_vector_type(2)));
 // fp32 input rows in the global address space (global, not flat, loads)
 typedef const __attribute__((address_space(1))) float* GlobalF;
 typedef __attribute__((address_space(1))) uint8_t* GlobalU8;
+
+// row[k .. k + 3] of a row of `cols` floats with no more than the alignment of
+// a float (what lies past the row's end is unspecified): one 16-byte load at
+// the last place in the row where it fits, and a shift where that is not k.
+__device__ __forceinline__ float4 load4_any(GlobalF row, int k, int cols) {
+  typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+  if (cols < 4)  // uniform
+    return make_float4(row[k < cols ? k : 0], row[k + 1 < cols ? k + 1 : 0],
+                       row[k + 2 < cols ? k + 2 : 0], 0.0f);
+  const int at = k < cols - 4 ? k : cols - 4, d = k - at;
+  const f32x4_a4 t = *reinterpret_cast<const __attribute__((address_space(1))) f32x4_a4*>(row + at);
+  return make_float4(d == 0 ? t.x : d == 1 ? t.y : d == 2 ? t.z : t.w, d == 0 ? t.y : d == 1 ? t.z : t.w,
+                     d == 0 ? t.z : t.w, t.w);
+}
 typedef __attribute__((address_space(3))) uint8_t* LdsU8;
 
 // Three-term splits hold FP6 (E2M3) terms: 0.75 byte per term and element
