@@ -100,3 +100,19 @@ def test_format_gemm_non_finite_inputs(gpu, fmt):
     fits = np.isfinite(top)
     assert rel_l2(y[36][fits] / 1e38, top[fits] / 1e38) <= 2e-6
     assert np.array_equal(y[36][~fits], top[~fits])
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("batch,inp,out", [
+    (6, 768, 448),    # below 8 rows, few products: the per-row kernel
+    (7, 8192, 40),    # long rows, few of them: likewise
+    (16, 512, 130),   # 4 waves
+    (16, 1024, 513),  # 8 waves; one weight row past a block
+    (17, 1024, 512),  # one batch row in the second block
+    (100, 768, 160),  # 7 batch blocks, the last with 4 rows
+    (33, 2048, 400),  # 16 waves, 3 batch blocks
+    (40, 2048, 1360),  # 85 x 3 blocks, the last count below 256
+    (40, 2048, 1376),  # 86 x 3: the split and the larger tiles
+])
+def test_format_small_products_match_f64(gpu, fmt, batch, inp, out):
+    test_format_gemm_matches_f64(gpu, fmt, batch, inp, out)

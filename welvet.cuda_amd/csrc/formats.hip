@@ -1385,26 +1385,27 @@ __global__ __launch_bounds__(64 * W) void k_fmt_gemm(FmtArgs a, FmtArgs plain,
   }
 }
 
-// At most 16 batch rows in one launch: a workgroup owns 16 weight rows and
-// all the batch rows, its W waves split the sub-blocks, x is split by the wave
+// Small batches in one launch: a workgroup owns 16 weight rows and 16 batch
+// rows (blockIdx.y), its W waves split the sub-blocks, x is split by the wave
 // itself (v_mfma_f32_16x16x32_bf16: lane l holds elements 8 (l / 16) .. + 7 of
 // batch row, and of weight row, l % 16; one product per term and sub-block,
 // two with the other half zeroed for fmt_halves). Bound by the latency of its
 // loads: those of `kDepth` sub-blocks are issued before the first of them is
 // used, and 16 waves make it two rounds at 4096 columns. 4096 x 4096 Q4_0 at 8
 // rows 10.2 us (13.0 on the fp32 matrix products), at 4 rows 9.6 us (11.6 with
-// every batch row streaming the weights); from row-major weights 14.9.
+// every batch row streaming the weights); from row-major weights 14.9. Fewer
+// sub-blocks feed fewer waves (rows_w).
 template <int FMT, int W>
 __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, int batch) {
   constexpr bool HALVES = fmt_halves(FMT), AFFINE = fmt_affine(FMT);
   constexpr int kDepth = 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
   const FmtRow row = fmt_row(a, n0 + i16 < a.rows ? n0 + i16 : a.rows - 1);
   const int t0 = (int)((int64_t)a.nsub * wave / W), t1 = (int)((int64_t)a.nsub * (wave + 1) / W);
-  const bool live = i16 < batch;
-  const float* src = a.x + (size_t)(live ? i16 : 0) * a.x_stride + 8 * g;
+  const bool live = m0 + i16 < batch;
+  const float* src = a.x + (size_t)(live ? m0 + i16 : 0) * a.x_stride + 8 * g;
   v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
   const bf16x8 zero = (bf16x8)(__bf16)0.0f;
 
@@ -1480,12 +1481,12 @@ __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, i
   // element r of lane (column i, group g) is batch row 4 g + r, weight row i
   for (int i = threadIdx.x; i < 256; i += 64 * W) {
     const int j = i >> 4, o = n0 + (i & 15);
-    if (j >= batch || o >= a.rows) continue;
+    if (m0 + j >= batch || o >= a.rows) continue;
     const int l = (j >> 2) * 16 + (i & 15), r = j & 3;
     float v = part[0][l][r];
 #pragma unroll
     for (int w = 1; w < W; ++w) v += part[w][l][r];
-    fmt_store<FMT>(plain, j, o, v);
+    fmt_store<FMT>(plain, m0 + j, o, v);
   }
 }
 
@@ -1498,8 +1499,18 @@ FmtArgs tile_weights(FmtArgs a, const FmtTiles& f) {
 
 template <int FMT, int W>
 Status rows_t(const FmtArgs& a, const FmtTiles& f, int batch, hipStream_t st) {
-  k_fmt_rows<FMT, W><<<(unsigned)((a.rows + 15) / 16), 64 * W, 0, st>>>(tile_weights(a, f), a, batch);
+  const dim3 grid((unsigned)((a.rows + 15) / 16), (unsigned)((batch + 15) / 16));
+  k_fmt_rows<FMT, W><<<grid, 64 * W, 0, st>>>(tile_weights(a, f), a, batch);
   return hip_status(hipGetLastError(), "format rows launch");
+}
+
+// Waves by the sub-blocks they split, 8 rows of Q4_0, us with 4 / 8 / 16 waves:
+// 512 x 256 4.1 / 4.1 / 5.4 (Q4_K 3.9 / 4.7 / 6.6), 1024 x 1024 4.5 / 4.1 / 5.5, 768 x 6400 6.0 / 5.7 /
+// 9.2, 2048 x 2048 6.8 / 5.8 / 5.6, 2048 x 4096 6.8 / 5.9 / 5.7.
+template <int FMT>
+Status rows_w(const FmtArgs& a, const FmtTiles& f, int batch, hipStream_t st) {
+  if (a.nsub <= 16) return rows_t<FMT, 4>(a, f, batch, st);
+  return a.nsub < 64 ? rows_t<FMT, 8>(a, f, batch, st) : rows_t<FMT, 16>(a, f, batch, st);
 }
 
 template <int FMT, int TM, int TN, int W>
@@ -1545,7 +1556,22 @@ Status gemv_w(const FmtArgs& a, int batch, int waves, hipStream_t st) {
 template <int FMT>
 Status gemv_f(const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws, size_t ws_bytes,
               hipStream_t st) {
-  if (batch >= format_rows_batch(FMT) && batch <= 16) return rows_t<FMT, 16>(a, f, batch, st);
+  // The per-row kernel's time goes with the rows times batch rows times chunks of
+  // 64 sub-blocks (partly filled ones count whole), the matrix-core kernel's
+  // with the sub-blocks that one workgroup walks. us, per-row / matrix cores
+  // (Q4_0 and Q6_K): 768 x 448 at 6 rows 3.7 / 4.1 and 3.9 / 4.6, 2048 x 2048 at 4
+  // rows 4.9 / 5.5 and 5.4 / 6.7, 768 x 6400 at 4 rows 7.7 / 5.5 and 11.1 / 6.6,
+  // 8192 x 256 at 6 rows 4.8 / 14.6 and 5.3 / 19.4. Only below 8 rows: from there
+  // an infinity of x meets each dequantized weight (fmt_store), where the
+  // per-row kernel's offset sums make it NaN.
+  const int chunks = (a.nsub + 63) / 64;
+  const int64_t per_row = (int64_t)a.rows * batch * chunks;
+  const bool small = batch < 8 && per_row <= (a.nsub > 40 ? 200 * (int64_t)a.nsub : 8192);
+  // Above 16 batch rows the split and the larger tiles are two launches (6.8 us
+  // at the least): one as long as every workgroup has a CU to itself.
+  const int64_t blocks = ((int64_t)a.rows + 15) / 16 * ((batch + 15) / 16);
+  if (!small && batch >= format_rows_batch(FMT) && (batch <= 16 || blocks <= 256))
+    return rows_w<FMT>(a, f, batch, st);
   if (batch > 16 && ws) {
     // as many rows at a time as the workspace holds terms of
     const size_t unit = (size_t)a.nsub * fmt_split_bytes(fmt_affine(FMT));
@@ -1561,7 +1587,6 @@ Status gemv_f(const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws, size_
   }
   // one wave per 64-sub-block chunk up to 4; then rows per group so that the
   // grid has >= 8 waves per CU when it can
-  const int chunks = (a.nsub + 63) / 64;
   const int waves = chunks <= 1 ? 1 : chunks == 2 ? 2 : 4;
   const long groups8 = ((long)a.rows + 7) / 8 * batch;
   if (groups8 * waves >= 8L * 256) return gemv_w<FMT, 8>(a, batch, waves, st);
