@@ -1,0 +1,28 @@
+"""The launch rules on the host: which sizes take which kernel."""
+import launch_rules
+
+CUS = 256
+
+
+def test_wide_tiles_do_not_leave_half_a_round_empty():
+    """Two rounds of wide tiles, each at least 1.5 narrow tiles' time, are kept
+    only where they are shorter than the rounds of twice as many narrow tiles."""
+    L = launch_rules.lib()
+    for tiles_m in (1, 8, 16, 17, 28, 32, 40, 64):
+        for cols in range(1, 49):
+            tiles = tiles_m * cols
+            wide = L.rule_mxg_wide(1, tiles_m, 256 * cols, 1, 0, 1024)
+            if tiles < CUS:
+                assert not wide
+                continue
+            rounds_wide, rounds_narrow = -(-tiles // CUS), -(-2 * tiles // CUS)
+            if rounds_wide == 2:
+                assert wide == (1.5 * rounds_wide < rounds_narrow)
+            else:
+                assert wide
+    # the joined projections of 8 x 512 tokens, 16 heads of 64
+    assert not L.rule_mxg_wide(1, 32, 3072, 1, 0, 1024)
+    assert not L.rule_mxg_wide(1, 32, 3072, 1, 1, 1024)
+    assert L.rule_mxg_wide(1, 32, 3072, 1, 1, 4096)  # FP4, long rows
+    assert not L.rule_mxg_wide(1, 32, 3072 + 128, 1, 0, 1024)  # no multiple of the width
+    assert L.rule_mxg_wide(64, 2, 1024, 1, 0, 1024)  # 64 members: two full rounds

@@ -28,6 +28,7 @@
 #include "act.h"
 #include "common.h"
 #include "kernels.h"
+#include "rules.h"
 #include "runtime.h"
 #include "split.h"
 
@@ -181,14 +182,6 @@ constexpr int kBM = 128;
 // waves per large-tile workgroup: 8 = two per SIMD, so one wave's MFMAs run
 // while the other waits on memory
 constexpr int kMxgWaves = 8;
-
-// Wide tiles (256 staged weight rows per step) move half the activation
-// bytes per MFMA; taken when they still give every CU a workgroup and N is a
-// multiple of their width (the weight rows and scales are padded to 128).
-bool mxg_wide(int members, int tiles_m, int N, int mats) {
-  const int bn = 256 / mats;
-  return N % bn == 0 && (long)members * tiles_m * (N / bn) >= 256;
-}
 
 // A grouped member's argument block, read field by field through the constant
 // address space: scalar loads into SGPRs (copying the struct as a whole
@@ -1621,7 +1614,7 @@ Status launch_t(const MxgArgs& p, int bm, hipStream_t st) {
         return hip_status(hipGetLastError(), "mxg K-split launch");
       }
     }
-    const bool wide = mxg_wide(1, tiles_m, p.N, MATS);
+    const bool wide = mxg_wide(1, tiles_m, p.N, MATS, DT == kFP4, p.kpad);
     const int tiles_n = wide ? (p.N + 256 / MATS - 1) / (256 / MATS) : (p.N + 128 / MATS - 1) / (128 / MATS);
     const unsigned grid = (unsigned)(tiles_m * tiles_n);
     if constexpr (MATS == 1) {
@@ -1751,7 +1744,7 @@ Status launch_split_group(const SplitJob* jobs, int n, bool vec, int x_stride, i
 template <int DT, bool BLK, int MATS>
 Status launch_group_t(const MxgArgs* tab, const MxgArgs& p, int n, hipStream_t st) {
   const int tiles_m = p.mpad / kBM;
-  const bool wide = mxg_wide(n, tiles_m, p.N, MATS);
+  const bool wide = mxg_wide(n, tiles_m, p.N, MATS, DT == kFP4, p.kpad);
   const int tiles_n = wide ? (p.N + 256 / MATS - 1) / (256 / MATS) : (p.N + 128 / MATS - 1) / (128 / MATS);
   const unsigned grid = (unsigned)(n * tiles_m * tiles_n);
   if constexpr (MATS == 1) {
