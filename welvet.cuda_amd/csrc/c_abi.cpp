@@ -57,6 +57,7 @@ hipStream_t pick(void* stream, hipStream_t own) {
 }  // namespace
 
 struct welvet_swiglu_session {
+  wv::HostSession host;
   wv::Stream stream;
   wv::SwiGLULayer layer;
   wv::Workspace ws;
@@ -65,6 +66,7 @@ struct welvet_swiglu_session {
 };
 
 struct welvet_mha_session {
+  wv::HostSession host;
   wv::Stream stream;
   wv::MHALayer layer;
   wv::Workspace ws;

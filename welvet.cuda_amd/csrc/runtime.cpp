@@ -39,7 +39,6 @@ std::string device_name() {
 // Pinned staging: two buffers, so the host copy of one chunk overlaps the
 // DMA of the other.
 constexpr size_t kStageBytes = 8u << 20;
-constexpr size_t kHostCallBytes = kStageBytes;
 std::mutex g_stage_mu;
 void* g_stage[2] = {nullptr, nullptr};
 hipEvent_t g_stage_ev[2] = {nullptr, nullptr};
@@ -52,7 +51,78 @@ Status stage_ready() {
   }
   return Status::ok();
 }
+
+// Pinned blocks of host_call, one per call in flight, allocated when first
+// needed and grown to the largest call that used them: at most 16 MiB each. The
+// first stays for the next session, as the staging buffers do; the others are
+// freed with the last session. Calls beyond kHostBlocks take staged copies.
+constexpr size_t kHostCallBytes = 8u << 20;  // x; and pre with post
+constexpr int kHostBlocks = 4;
+struct HostBlock {
+  void* p = nullptr;
+  size_t bytes = 0;
+  bool used = false;
+};
+std::mutex g_host_mu;
+HostBlock g_host[kHostBlocks];
+int g_host_sessions = 0;
+
+// A block of at least n bytes for the holder's lifetime; p is null when all are
+// in use or the memory cannot be had. The lock covers the choice alone.
+struct HostLoan {
+  void* p = nullptr;
+  explicit HostLoan(size_t n) {
+    {
+      std::lock_guard<std::mutex> lock(g_host_mu);
+      for (HostBlock& b : g_host)
+        if (!b.used) {
+          block_ = &b;
+          b.used = true;
+          break;
+        }
+    }
+    if (!block_) return;
+    if (block_->bytes < n) {
+      size_t size = 64u << 10;
+      while (size < n) size *= 2;
+      free_block(block_);
+      if (hipHostMalloc(&block_->p, size, hipHostMallocDefault) == hipSuccess) {
+        block_->bytes = size;
+      } else {
+        (void)hipGetLastError();
+        block_->p = nullptr;
+      }
+    }
+    p = block_->p;
+  }
+  ~HostLoan() {
+    if (!block_) return;
+    std::lock_guard<std::mutex> lock(g_host_mu);
+    block_->used = false;
+  }
+  HostLoan(const HostLoan&) = delete;
+  HostLoan& operator=(const HostLoan&) = delete;
+  static void free_block(HostBlock* b) {
+    if (b->p && hipHostFree(b->p) != hipSuccess) (void)hipGetLastError();
+    b->p = nullptr, b->bytes = 0;
+  }
+
+ private:
+  HostBlock* block_ = nullptr;
+};
 }  // namespace
+
+HostSession::HostSession() {
+  std::lock_guard<std::mutex> lock(g_host_mu);
+  ++g_host_sessions;
+}
+
+HostSession::~HostSession() {
+  std::lock_guard<std::mutex> lock(g_host_mu);
+  if (--g_host_sessions > 0) return;
+  for (int i = 1; i < kHostBlocks; ++i)
+    if (!g_host[i].used) HostLoan::free_block(&g_host[i]);
+}
 
 Status init_device() {
   std::lock_guard<std::mutex> lock(g_mu);
@@ -173,21 +243,18 @@ Status copy_d2h(void* dst, const void* src, size_t n, hipStream_t st) {
 Status host_call(const void* x, void* dx, size_t xb, void* pre, const void* dpre, size_t yb,
                  void* post, const void* dpost, size_t zb, hipStream_t st,
                  const std::function<Status()>& run) {
-  // Small calls: x and the outputs go through the staging buffers (x the
-  // first, the outputs the second) by kernels on the call's own stream, and
-  // the host waits once, at the end. A copy_h2d and two copy_d2h wait three
-  // times more and pass from the copy engine to the kernels and back.
-  // `run` only launches work: it makes no staged copy (the lock is held).
-  // Calls that find the buffers in use take the copies, which wait for them.
-  const size_t at = (size_t)round_up((int64_t)yb, 256);
-  if (xb <= kHostCallBytes && at + zb <= kHostCallBytes) {
-    std::unique_lock<std::mutex> lock(g_stage_mu, std::try_to_lock);
-    if (lock.owns_lock()) {
-      WV_TRY(stage_ready());
-      char* in = static_cast<char*>(g_stage[0]);
-      char* out = static_cast<char*>(g_stage[1]);
-      // the next caller refills the buffers: the stream is drained on every
-      // way out of here
+  // Small calls: x and the outputs go through a pinned block by kernels on the
+  // call's own stream, and the host waits once, at the end, under no lock. A
+  // copy_h2d and two copy_d2h wait three times more and pass from the copy
+  // engine to the kernels and back.
+  const size_t pre_at = (size_t)round_up((int64_t)xb, 256);
+  const size_t post_at = pre_at + (size_t)round_up((int64_t)yb, 256);
+  if (xb <= kHostCallBytes && post_at - pre_at + zb <= kHostCallBytes) {
+    HostLoan loan(post_at + zb);
+    if (loan.p) {
+      char* buf = static_cast<char*>(loan.p);
+      // the block's next user refills it: the stream is drained on every way
+      // out of here
       struct Drain {
         hipStream_t st;
         bool done = false;
@@ -195,14 +262,14 @@ Status host_call(const void* x, void* dx, size_t xb, void* pre, const void* dpre
           if (!done && hipStreamSynchronize(st) != hipSuccess) (void)hipGetLastError();
         }
       } drain{st};
-      std::memcpy(in, x, xb);
-      WV_TRY(launch_copy({dx, in, xb}, {}, st));
+      std::memcpy(buf, x, xb);
+      WV_TRY(launch_copy({dx, buf, xb}, {}, st));
       WV_TRY(run());
-      WV_TRY(launch_copy({out, dpre, yb}, {out + at, dpost, zb}, st));
+      WV_TRY(launch_copy({buf + pre_at, dpre, yb}, {buf + post_at, dpost, zb}, st));
       drain.done = true;
       WV_HIP(hipStreamSynchronize(st));
-      std::memcpy(pre, out, yb);
-      std::memcpy(post, out + at, zb);
+      std::memcpy(pre, buf + pre_at, yb);
+      std::memcpy(post, buf + post_at, zb);
       return Status::ok();
     }
   }

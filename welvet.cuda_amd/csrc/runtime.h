@@ -24,9 +24,19 @@ int cu_count();
 Status copy_h2d(void* dst, const void* src, size_t n, hipStream_t st);
 Status copy_d2h(void* dst, const void* src, size_t n, hipStream_t st);
 
+// Held by a session whose calls may go through host_call: the pinned blocks
+// that calls in flight at once needed are freed with the last one.
+struct HostSession {
+  HostSession();
+  ~HostSession();
+  HostSession(const HostSession&) = delete;
+  HostSession& operator=(const HostSession&) = delete;
+};
+
 // One forward call on host buffers: x (xb bytes) to dx, `run` queued on `st`,
 // then pre and post (yb and zb bytes) from dpre and dpost; complete on return.
-// Device buffers are 16-byte aligned and sizes are whole floats.
+// Device buffers are 16-byte aligned and sizes are whole floats. Calls of
+// different threads overlap.
 Status host_call(const void* x, void* dx, size_t xb, void* pre, const void* dpre, size_t yb,
                  void* post, const void* dpost, size_t zb, hipStream_t st,
                  const std::function<Status()>& run);

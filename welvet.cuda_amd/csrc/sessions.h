@@ -10,6 +10,7 @@
 // Dense session: one layer mounted at a fixed batch, its stream, workspace
 // and the device buffers of the host-buffer execute.
 struct welvet_dense_session {
+  wv::HostSession host;
   wv::Stream stream;
   wv::DenseLayer layer;
   wv::Workspace ws;
