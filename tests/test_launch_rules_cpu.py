@@ -1,4 +1,6 @@
 """The launch rules on the host: which sizes take which kernel."""
+import ctypes
+
 import launch_rules
 
 CUS = 256
@@ -26,3 +28,14 @@ def test_wide_tiles_do_not_leave_half_a_round_empty():
     assert L.rule_mxg_wide(1, 32, 3072, 1, 1, 4096)  # FP4, long rows
     assert not L.rule_mxg_wide(1, 32, 3072 + 128, 1, 0, 1024)  # no multiple of the width
     assert L.rule_mxg_wide(64, 2, 1024, 1, 0, 1024)  # 64 members: two full rounds
+
+
+def test_joined_projections_stay_within_the_large_tiles():
+    """Three matrices below 2 GiB each whose joined rows reach it: mha_join, which
+    asks this rule, must leave them apart (the product refuses the joined one)."""
+    fit = launch_rules.lib().rule_mxg_weights_fit
+    fit.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
+    d = 26880  # FP8, full heads
+    assert fit(d, d) and not fit(3 * d, d)
+    assert fit(3 * 26624, 26624) and not fit(3 * 26880, 26880)
+    assert fit((1 << 31) // 32768 - 256, 32768) and not fit((1 << 31) // 32768 - 255, 32768)

@@ -13,6 +13,7 @@
 #include <cstring>
 
 #include "codec.h"
+#include "rules.h"
 
 namespace wv {
 
@@ -970,6 +971,9 @@ Status mha_join(MHALayer* L, hipStream_t st) {
       return Status::ok();
     rows += p->out;
   }
+  // three matrices that fit the large-tile product one by one stay apart where
+  // the joined one would not
+  if (!mxg_weights_fit(rows, d0.pitch)) return Status::ok();
   DenseLayer& J = L->qkv;
   DeviceWeights& j = J.dev;
   J.in = L->q.in, J.act = kLinear, J.terms = L->q.terms;

@@ -1576,7 +1576,7 @@ Status launch_t(const MxgArgs& p, int bm, hipStream_t st) {
     return Status::err(kInvalid, "mxg: RoPE epilogue needs the large tiles, one matrix, no epilogue");
   if (bm == kBM) {
     if ((size_t)kTerms * p.mpad * p.kpad >= (1ull << 31) ||
-        (size_t)round_up(p.N, 256) * p.pitch >= (1ull << 31))
+        !mxg_weights_fit(p.N, p.pitch))
       return Status::err(kUnsupported, "mxg: operands above 2 GiB");
     const int tiles_m = p.mpad / kBM;
     // with p.next set, a K split ends in the reduce that also writes the
@@ -1785,7 +1785,7 @@ Status launch_mxg_group(const MxgArgs* tab, const MxgArgs& p, int n, int dtype, 
   if (mxg_block_m(p.M) != kBM || p.mpad % kBM != 0 || p.kpad % 256 != 0)
     return Status::err(kInvalid, "mxg group: needs the large-tile layout");
   if ((size_t)kTerms * p.mpad * p.kpad >= (1ull << 31) ||
-      (size_t)round_up(p.N, 256) * p.pitch >= (1ull << 31))
+      !mxg_weights_fit(p.N, p.pitch))
     return Status::err(kUnsupported, "mxg: operands above 2 GiB");
   const bool two = p.mats == 2;
   switch (dtype) {

@@ -27,4 +27,10 @@ inline bool mxg_wide(int members, int tiles_m, int N, int mats, bool fp4, int kp
   return !half_empty || (fp4 && kpad > 1536);
 }
 
+// The large-tile product addresses its weight codes with 32-bit offsets: N rows
+// (padded to a wide tile) of `pitch` bytes stay below 2 GiB.
+inline bool mxg_weights_fit(int64_t N, int64_t pitch) {
+  return (N + 255) / 256 * 256 * pitch < (1ll << 31);
+}
+
 }  // namespace wv
