@@ -99,3 +99,26 @@ def test_non_finite_token_stays_with_the_queries_that_see_it(gpu, oracle, bad, h
     assert np.isfinite(attn[:t]).all()
     assert rel_l2(attn[:t], clean[:t]) <= 3e-6
     assert not np.isfinite(attn[t:, 5]).any()
+
+
+@pytest.mark.parametrize("B,S,msl", [(40, 1, 1), (64, 1, 2), (40, 2, 2), (40, 3, 4), (60, 4, 4),
+                                     (30, 8, 8), (20, 15, 15), (20, 16, 16)])
+@pytest.mark.parametrize("H,hd", [(1, 64), (2, 32), (1, 128)])
+@pytest.mark.parametrize("mask", [CAUSAL, FULL])
+def test_short_alibi_rings_keep_their_digits(gpu, oracle, B, S, msl, H, hd, mask):
+    """Rings of a few rows that each stand for many positions, under the flattest
+    slopes (2^-8, with two heads also 2^-4): the sum over a row's positions is
+    r^c - 1 over r - 1 with r near 1. Inputs of +-1, so an output's error is that of
+    the weights. Bound: exponents of a few units rounded to f32 (2^-24 of 4 is
+    2.4e-7) and weights of 2^-23, together 3.6e-7 of weights that sum to 1; with 1 - r
+    formed in f32 it was 2e-6."""
+    rng = np.random.default_rng(B + S + hd)
+    Q, K, V, O, _ = layer(B + hd, B, S, H, H, hd)
+    d = H * hd
+    x = rng.choice(np.float32([-1, 1]), size=(B * S, d))
+    attn, _ = cxx_probe.mha_masked(B, S, d, H, H, msl, mask, ALIBI, 0, 1, 0, 0, 4, Q, K, V, O, x)
+    want = oracle.mha_attention(x @ Q.T, x @ K.T, x @ V.T, B, S, H, H, hd, msl, mask, ALIBI, 0, 0, 0,
+                                1, threads=8)
+    err = float(np.max(np.abs(attn - want)))
+    print(f"ring of {msl}, {B} x {S}, {H} x {hd}: largest error {err:.2e}")
+    assert err <= 3.6e-7

@@ -272,26 +272,38 @@ __device__ __forceinline__ int key_count(const AttnArgs& a, int p, int qp, int l
   return c + 1;
 }
 
+// ALiBi over rings of fewer than kShortRing rows: 1 - r, formed in f32 with r =
+// e^(-s msl) near 1, keeps too few digits at the flattest slope (2^-8): 4e-6 of a
+// weight at 2 rows, from 16 on below the exponents' own rounding. SHORT takes
+// r^c - 1 over r - 1 from expm1f instead, in kernels of its own (expm1f in the
+// others costs them up to 7%, in registers also where it is not run).
+constexpr int kShortRing = 16;
+
 // The ALiBi constants of a head: the slope in log2 units and, for the sums
-// over a row's positions, -log2(1 - r).
+// over a row's positions, x = log2 r and lginv = -log2(1 - r); SHORT: x = ln r
+// and lginv = 1 / (r - 1).
 struct Bias {
   float sl2, x, lginv;
 };
 
 // log2(1 + r + ... + r^(c - 1)); log2(c) without ALiBi.
+template <bool SHORT>
 __device__ __forceinline__ float log2_copies(int c, const Bias& s) {
+  if constexpr (SHORT)
+    return c <= 1 ? 0.0f : __builtin_amdgcn_logf(expm1f(s.x * (float)c) * s.lginv);
   if (s.sl2 == 0.0f) return __builtin_amdgcn_logf((float)c);
   return __builtin_amdgcn_logf(1.0f - __builtin_amdgcn_exp2f(s.x * (float)c)) + s.lginv;
 }
 
 // log2 of the weight that row p's positions add to e^score for query qp;
 // -inf when none is allowed.
+template <bool SHORT>
 __device__ __forceinline__ float log2_weight(const AttnArgs& a, int p, int qp, int last, int lo,
                                              int hi, float inv_msl, const Bias& s) {
   int first, above;
   const int c = key_count(a, p, qp, last, lo, hi, inv_msl, first, above);
   if (s.sl2 == 0.0f) return __builtin_amdgcn_logf((float)(c + above));  // log2(0) = -inf
-  const float below = c > 0 ? fmaf(-s.sl2, (float)(qp - first), log2_copies(c, s)) : -INFINITY;
+  const float below = c > 0 ? fmaf(-s.sl2, (float)(qp - first), log2_copies<SHORT>(c, s)) : -INFINITY;
   if (!above) return below;
   const float up = -s.sl2 * (float)(p - qp);
   const float m = fmaxf(up, below);
@@ -322,7 +334,7 @@ __device__ __forceinline__ v4f mfma_terms(const bf16x8 (&a)[T], const bf16x8 (&b
   return acc;
 }
 
-template <int HD, bool SIG, bool GEN, int WAVES>
+template <int HD, bool SIG, bool GEN, int WAVES, bool SHORT = false>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? (GEN && HD > 64 ? 1 : 2) : WAVES / 4, 8)))
 void k_attn_mfma(AttnArgs a, int qblocks) {
   constexpr int KT = attn_keys(HD, GEN, WAVES);         // keys per tile
@@ -364,8 +376,13 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
     inv_msl = 1.0f / (float)a.msl;
     if (a.alibi) {
       al.sl2 = (float)(exp2(-(double)(h + 1) * 8.0 / (double)a.heads) * 1.4426950408889634);
-      al.x = -al.sl2 * (float)a.msl;
-      al.lginv = -__builtin_amdgcn_logf(1.0f - __builtin_amdgcn_exp2f(al.x));
+      if constexpr (SHORT) {
+        al.x = (float)(-exp2(-(double)(h + 1) * 8.0 / (double)a.heads) * (double)a.msl);
+        al.lginv = 1.0f / expm1f(al.x);
+      } else {
+        al.x = -al.sl2 * (float)a.msl;
+        al.lginv = -__builtin_amdgcn_logf(1.0f - __builtin_amdgcn_exp2f(al.x));
+      }
     }
   }
 
@@ -570,7 +587,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
       if (GEN && cu > 0) {
         // ALiBi: the distance to the row's first position, then the sum over
         // its cu positions as one factor (log2_copies)
-        const float lc = log2_copies(cu, al);
+        const float lc = log2_copies<SHORT>(cu, al);
         const float d0 = (float)(qp - first0 - 4 * g);
 #pragma unroll
         for (int kb = 0; kb < NB; ++kb)
@@ -585,7 +602,7 @@ void k_attn_mfma(AttnArgs a, int qblocks) {
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float bias = log2_weight(a, t0 + 16 * kb + 4 * g + i, qp, last, lo, hi, inv_msl, al);
+            const float bias = log2_weight<SHORT>(a, t0 + 16 * kb + 4 * g + i, qp, last, lo, hi, inv_msl, al);
             w[4 * kb + i] = bias > -INFINITY ? fmaf(sc[kb][i], scale_log2, bias) : -INFINITY;
             smax = fmaxf(smax, w[4 * kb + i]);
           }
@@ -758,17 +775,21 @@ bool attention_writes_split(const AttnArgs& a) {
   return attention_fast(a) && (a.heads * a.hd) % 256 == 0 && a.seq % 16 == 0;
 }
 
-template <int HD, bool SIG, bool GEN, int WAVES>
+template <int HD, bool SIG, bool GEN, int WAVES, bool SHORT = false>
 static void attn_launch(const AttnArgs& a, hipStream_t st) {
   const int qblocks = (a.seq + 16 * WAVES - 1) / (16 * WAVES);
   const dim3 grid((unsigned)(a.tokens / a.seq * qblocks), (unsigned)a.heads);
-  k_attn_mfma<HD, SIG, GEN, WAVES><<<grid, 64 * WAVES, 0, st>>>(a, qblocks);
+  k_attn_mfma<HD, SIG, GEN, WAVES, SHORT><<<grid, 64 * WAVES, 0, st>>>(a, qblocks);
 }
 
 template <int HD, bool GEN>
 static void attn_waves_of(const AttnArgs& a, hipStream_t st) {
   constexpr int most = HD <= 64 ? 16 : 8;
   if (a.sigmoid) return attn_launch<HD, true, GEN, most>(a, st);
+  if constexpr (GEN) {
+    // (a ring holds the sequence: one wave has all of its queries)
+    if (a.alibi && a.msl < kShortRing) return attn_launch<HD, false, true, 4, true>(a, st);
+  }
   const auto groups = [&](int waves) {
     return (int64_t)(a.tokens / a.seq) * a.heads * ((a.seq + 16 * waves - 1) / (16 * waves));
   };
