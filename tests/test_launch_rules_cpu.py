@@ -39,3 +39,41 @@ def test_joined_projections_stay_within_the_large_tiles():
     assert fit(d, d) and not fit(3 * d, d)
     assert fit(3 * 26624, 26624) and not fit(3 * 26880, 26880)
     assert fit((1 << 31) // 32768 - 256, 32768) and not fit((1 << 31) // 32768 - 255, 32768)
+
+
+FORMATS = [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 16, 17]
+
+
+def test_format_waves_load_what_they_have():
+    """The runs of sub-blocks that a wave of the small-batch kernel loads ahead:
+    a built (waves, depth), and less than one sub-block per run past its last."""
+    built = {(4, 2), (4, 3), (4, 4), (8, 3), (8, 4), (16, 3), (16, 4)}
+    seen = set()
+    for nsub in range(1, 400):
+        p = launch_rules.format_plan(2, 16, 32 * nsub, 16)
+        assert p.kernel == launch_rules.ROWS
+        seen.add((p.waves, p.depth))
+        per = -(-nsub // p.waves)
+        runs = -(-per // p.depth)
+        assert runs * p.depth - per < max(runs, 3 - per)  # (2 is the least depth)
+    assert seen == built
+
+
+def test_format_kernels_by_size():
+    plan = launch_rules.format_plan
+    for fmt in FORMATS:
+        for batch in (1, 2, 3):
+            assert plan(fmt, 4096, 4096, batch).kernel == launch_rules.PER_ROW
+        for out, inp in ((256, 512), (8192, 256), (448, 768), (4096, 4096)):
+            assert plan(fmt, out, inp, 8).kernel == plan(fmt, out, inp, 16).kernel == launch_rules.ROWS
+        # narrow inputs at many rows: one launch while it is the shorter one
+        assert plan(fmt, 256, 512, 300).kernel == launch_rules.ROWS
+        assert plan(fmt, 256, 512, 1000).kernel == launch_rules.ROWS
+        assert plan(fmt, 448, 768, 300).kernel == launch_rules.ROWS
+        assert plan(fmt, 8192, 256, 64).kernel == launch_rules.GEMM
+        assert plan(fmt, 1024, 1024, 100).kernel == launch_rules.ROWS
+        assert plan(fmt, 1024, 1024, 300).kernel == launch_rules.GEMM
+        assert plan(fmt, 4096, 4096, 17).kernel == launch_rules.GEMM
+        # (the grid's second dimension holds 65535 blocks of 16 batch rows)
+        assert plan(fmt, 16, 32, 1 << 20).kernel == launch_rules.GEMM
+        assert [plan(fmt, 4096, 4096, b)[3:5] for b in (64, 128, 256, 512)] == [(1, 1), (1, 2), (2, 2), (2, 4)]

@@ -978,11 +978,6 @@ constexpr bool fmt_halves(int fmt) { return fmt == kQ2_K || fmt == kQ3_K || fmt 
 constexpr int fmt_header(int fmt) {
   return fmt == kQ4_K || fmt == kQ5_K || fmt == kQ3_K ? 16 : fmt == kIQ4_XS ? 8 : 0;
 }
-constexpr bool fmt_affine(int fmt) {
-  return fmt == kQ4_1 || fmt == kQ5_1 || fmt == kQ2_K || fmt == kQ4_K || fmt == kQ5_K;
-}
-// operand bytes of 32 batch rows x 32 elements
-constexpr int fmt_split_bytes(bool affine) { return affine ? 7168 : 6144; }
 
 // v as three bf16 terms, each rounding the remainder of those before it.
 __device__ __forceinline__ void fmt_terms(float v, __bf16 (&t)[3]) {
@@ -1394,11 +1389,10 @@ __global__ __launch_bounds__(64 * W) void k_fmt_gemm(FmtArgs a, FmtArgs plain,
 // used, and 16 waves make it two rounds at 4096 columns. 4096 x 4096 Q4_0 at 8
 // rows 10.2 us (13.0 on the fp32 matrix products), at 4 rows 9.6 us (11.6 with
 // every batch row streaming the weights); from row-major weights 14.9. Fewer
-// sub-blocks feed fewer waves (rows_w).
-template <int FMT, int W>
+// sub-blocks feed fewer waves (format_plan).
+template <int FMT, int W, int kDepth>
 __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, int batch) {
   constexpr bool HALVES = fmt_halves(FMT), AFFINE = fmt_affine(FMT);
-  constexpr int kDepth = 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i16 = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
@@ -1497,20 +1491,25 @@ FmtArgs tile_weights(FmtArgs a, const FmtTiles& f) {
   return a;
 }
 
-template <int FMT, int W>
+template <int FMT, int W, int D>
 Status rows_t(const FmtArgs& a, const FmtTiles& f, int batch, hipStream_t st) {
   const dim3 grid((unsigned)((a.rows + 15) / 16), (unsigned)((batch + 15) / 16));
-  k_fmt_rows<FMT, W><<<grid, 64 * W, 0, st>>>(tile_weights(a, f), a, batch);
+  k_fmt_rows<FMT, W, D><<<grid, 64 * W, 0, st>>>(tile_weights(a, f), a, batch);
   return hip_status(hipGetLastError(), "format rows launch");
 }
 
-// Waves by the sub-blocks they split, 8 rows of Q4_0, us with 4 / 8 / 16 waves:
-// 512 x 256 4.1 / 4.1 / 5.4 (Q4_K 3.9 / 4.7 / 6.6), 1024 x 1024 4.5 / 4.1 / 5.5, 768 x 6400 6.0 / 5.7 /
-// 9.2, 2048 x 2048 6.8 / 5.8 / 5.6, 2048 x 4096 6.8 / 5.9 / 5.7.
 template <int FMT>
-Status rows_w(const FmtArgs& a, const FmtTiles& f, int batch, hipStream_t st) {
-  if (a.nsub <= 16) return rows_t<FMT, 4>(a, f, batch, st);
-  return a.nsub < 64 ? rows_t<FMT, 8>(a, f, batch, st) : rows_t<FMT, 16>(a, f, batch, st);
+Status rows_f(const FmtPlan& p, const FmtArgs& a, const FmtTiles& f, int batch, hipStream_t st) {
+  switch (p.waves * 10 + p.depth) {
+  case 42: return rows_t<FMT, 4, 2>(a, f, batch, st);
+  case 43: return rows_t<FMT, 4, 3>(a, f, batch, st);
+  case 44: return rows_t<FMT, 4, 4>(a, f, batch, st);
+  case 83: return rows_t<FMT, 8, 3>(a, f, batch, st);
+  case 84: return rows_t<FMT, 8, 4>(a, f, batch, st);
+  case 163: return rows_t<FMT, 16, 3>(a, f, batch, st);
+  case 164: return rows_t<FMT, 16, 4>(a, f, batch, st);
+  }
+  return Status::err(kInternal, "format rows: shape");
 }
 
 template <int FMT, int TM, int TN, int W>
@@ -1527,18 +1526,10 @@ Status gemm_f(const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws, hipSt
   const dim3 grid((unsigned)((a.nsub + 3) / 4), (unsigned)mblocks);
   k_fmt_split<fmt_affine(FMT)><<<grid, kThreads, 0, st>>>(a.x, a.x_stride, batch, a.nsub, ws);
   WV_HIP(hipGetLastError());
-  const auto tiles = [&](int tm, int tn) {
-    return (int64_t)((batch + 32 * tm - 1) / (32 * tm)) * ((a.rows + 32 * tn - 1) / (32 * tn));
-  };
-  // The largest tile (a decoded weight and a loaded term feed more products)
-  // that still reaches three quarters of the 256 CUs. 4096 x 4096 Q4_0, us at
-  // tiles 1 x 1 / 1 x 2 / 2 x 2 / 2 x 4: 64 rows 15.9 / 19.0 / 31.9 / 49.0, 128
-  // rows 26.6 / 22.1 / 34.1 / 49.3, 256 rows 50.4 / 39.7 / 40.1 / 52.5, 512 rows
-  // 114 / 75 / 74 / 62.
-  constexpr int64_t kFill = 192;
-  if (tiles(2, 4) >= kFill) return gemm_t<FMT, 2, 4, 8>(a, f, batch, ws, st);
-  if (tiles(2, 2) >= kFill) return gemm_t<FMT, 2, 2, 8>(a, f, batch, ws, st);
-  if (tiles(1, 2) >= kFill) return gemm_t<FMT, 1, 2, 8>(a, f, batch, ws, st);
+  const FmtTile t = format_tile(a.rows, batch);
+  if (t.tn == 4) return gemm_t<FMT, 2, 4, 8>(a, f, batch, ws, st);
+  if (t.tm == 2) return gemm_t<FMT, 2, 2, 8>(a, f, batch, ws, st);
+  if (t.tn == 2) return gemm_t<FMT, 1, 2, 8>(a, f, batch, ws, st);
   return gemm_t<FMT, 1, 1, 8>(a, f, batch, ws, st);
 }
 
@@ -1556,35 +1547,20 @@ Status gemv_w(const FmtArgs& a, int batch, int waves, hipStream_t st) {
 template <int FMT>
 Status gemv_f(const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws, size_t ws_bytes,
               hipStream_t st) {
-  // The per-row kernel's time goes with the rows times batch rows times chunks of
-  // 64 sub-blocks (partly filled ones count whole), the matrix-core kernel's
-  // with the sub-blocks that one workgroup walks. us, per-row / matrix cores
-  // (Q4_0 and Q6_K): 768 x 448 at 6 rows 3.7 / 4.1 and 3.9 / 4.6, 2048 x 2048 at 4
-  // rows 4.9 / 5.5 and 5.4 / 6.7, 768 x 6400 at 4 rows 7.7 / 5.5 and 11.1 / 6.6,
-  // 8192 x 256 at 6 rows 4.8 / 14.6 and 5.3 / 19.4. Only below 8 rows: from there
-  // an infinity of x meets each dequantized weight (fmt_store), where the
-  // per-row kernel's offset sums make it NaN.
-  const int chunks = (a.nsub + 63) / 64;
-  const int64_t per_row = (int64_t)a.rows * batch * chunks;
-  const bool small = batch < 8 && per_row <= (a.nsub > 40 ? 200 * (int64_t)a.nsub : 8192);
-  // Above 16 batch rows the split and the larger tiles are two launches (6.8 us
-  // at the least): one as long as every workgroup has a CU to itself.
-  const int64_t blocks = ((int64_t)a.rows + 15) / 16 * ((batch + 15) / 16);
-  if (!small && batch >= format_rows_batch(FMT) && (batch <= 16 || blocks <= 256))
-    return rows_w<FMT>(a, f, batch, st);
-  if (batch > 16 && ws) {
-    // as many rows at a time as the workspace holds terms of
-    const size_t unit = (size_t)a.nsub * fmt_split_bytes(fmt_affine(FMT));
-    const int64_t rows = (int64_t)(ws_bytes / unit) * 32;
-    for (int64_t j = 0; rows > 0 && j < batch; j += rows) {
+  const FmtPlan p = format_plan(FMT, a.rows, a.nsub, batch);
+  if (p.kernel == FmtKernel::kRows) return rows_f<FMT>(p, a, f, batch, st);
+  const int64_t run = ws ? format_run_rows(FMT, a.nsub, ws_bytes) : 0;
+  if (p.kernel == FmtKernel::kGemm && run > 0) {
+    for (int64_t j = 0; j < batch; j += run) {
       FmtArgs c = a;
       c.x = a.x + (size_t)j * a.x_stride;
       c.pre = a.pre + (size_t)j * a.out_stride;
       c.post = a.post ? a.post + (size_t)j * a.out_stride : nullptr;
-      WV_TRY(gemm_f<FMT>(c, f, (int)(batch - j < rows ? batch - j : rows), ws, st));
+      WV_TRY(gemm_f<FMT>(c, f, (int)(batch - j < run ? batch - j : run), ws, st));
     }
-    if (rows > 0) return Status::ok();
+    return Status::ok();
   }
+  const int chunks = (a.nsub + 63) / 64;
   // one wave per 64-sub-block chunk up to 4; then rows per group so that the
   // grid has >= 8 waves per CU when it can
   const int waves = chunks <= 1 ? 1 : chunks == 2 ? 2 : 4;
@@ -1710,12 +1686,6 @@ Status format_interleave(int fmt, const FmtArgs& a, uint8_t* buf, int rpad, FmtT
   const int hd = fmt_header(fmt);
   WV_TRY(array(a.s, hd ? a.nsub / 8 : a.nsub, hd ? hd : G.sb, &f->s));
   return array(a.e, a.nsub / 8, G.eb, &f->e);
-}
-
-size_t format_ws_bytes(int nsub, int batch) {
-  if (batch <= 16) return 0;
-  const size_t n = (size_t)((batch + 31) / 32) * nsub * fmt_split_bytes(true);
-  return n < kFmtWsBytes ? n : kFmtWsBytes;
 }
 
 Status launch_format_gemv(int fmt, const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws,

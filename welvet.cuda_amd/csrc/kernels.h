@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.h"
+#include "rules.h"
 
 namespace wv {
 
@@ -338,13 +339,6 @@ Status launch_sgd(const DeviceWeights& d, const double* dw, double lr, float* w_
 Status launch_dequant(const DeviceWeights& d, float* w, hipStream_t st);
 
 // ---- packed block formats (formats.hip) ----
-// QuantFormat ids: the reference's enum (include/welvet/weights.hpp:12-15)
-// holds only None; the other values follow the order of its format table
-// (README.md:361-383).
-enum QuantFormat : int32_t {
-  kFmtNone = 0, kQ8_0 = 1, kQ4_0 = 2, kQ4_1 = 3, kQ5_0 = 4, kQ5_1 = 5, kQ2_K = 6, kQ3_K = 7,
-  kQ4_K = 8, kQ5_K = 9, kQ6_K = 10, kIQ4_NL = 16, kIQ4_XS = 17, kFmtLast = 20
-};
 // Elements and packed bytes per block; bytes per 32-element sub-block of the
 // resident code (q), high-bit (h) and scale (s) arrays, and of the per-256
 // array e (Q6_K's d).
@@ -400,20 +394,11 @@ struct FmtTiles {
 size_t format_interleaved_bytes(int fmt, int rows, int nsub);
 Status format_interleave(int fmt, const FmtArgs& a, uint8_t* buf, int rpad, FmtTiles* f,
                          hipStream_t st);
-// Batch rows from which the matrix cores take the product. 4096 x 4096 at 4 and
-// 6 rows, us, the per-row kernel against the matrix cores: Q8_0 16.3 / 10.0 and
-// 21.7 / 10.4, Q4_0 11.6 / 9.8 and 13.8 / 10.1, Q4_1 10.1 / 11.6 and 13.8 /
-// 11.9, Q2_K 11.5 / 13.6 and 14.3 / 14.0 (the others like Q4_0).
-constexpr int format_rows_batch(int fmt) {
-  return fmt == kQ2_K ? 6 : fmt == kQ4_1 || fmt == kQ5_1 ? 5 : 4;
-}
 // y = W x for every one of `batch` rows of x (a.x, a.x_stride), with the Dense
 // epilogue into a.pre / a.post. f: the interleaved copy, if there is one. ws:
 // scratch for the product above 16 rows (format_ws_bytes, at most kFmtWsBytes,
 // beyond which it takes the rows in several runs); without it every batch
 // row streams the weights there.
-constexpr size_t kFmtWsBytes = 64ull << 20;
-size_t format_ws_bytes(int nsub, int batch);
 Status launch_format_gemv(int fmt, const FmtArgs& a, const FmtTiles& f, int batch, uint8_t* ws,
                           size_t ws_bytes, hipStream_t st);
 
