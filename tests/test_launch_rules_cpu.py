@@ -47,10 +47,10 @@ FORMATS = [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 16, 17]
 def test_format_waves_load_what_they_have():
     """The runs of sub-blocks that a wave of the small-batch kernel loads ahead:
     a built (waves, depth), and less than one sub-block per run past its last."""
-    built = {(4, 2), (4, 3), (4, 4), (8, 3), (8, 4), (16, 3), (16, 4)}
+    built = {(4, 2), (4, 3), (4, 4), (8, 3), (8, 4), (16, 2), (16, 3), (16, 4)}
     seen = set()
-    for nsub in range(1, 400):
-        p = launch_rules.format_plan(2, 16, 32 * nsub, 16)
+    for fmt, rows, nsub in [(f, r, n) for f in (2, 8) for r in (16, 8192) for n in range(1, 400)]:
+        p = launch_rules.format_plan(fmt, rows, 32 * nsub, 16)
         assert p.kernel == launch_rules.ROWS
         seen.add((p.waves, p.depth))
         per = -(-nsub // p.waves)

@@ -103,7 +103,11 @@ inline FmtPlan format_plan(int fmt, int rows, int nsub, int batch) {
     // 4: what a run holds past the last one is work for nothing (256 x 8192 at 16
     // rows, 2 sub-blocks a wave, with runs of 4 / 2: Q4_0 4.6 / 3.6, Q6_K 5.2 / 3.8;
     // 768 x 448, 3 a wave, with 4 / 3: Q6_K 4.9 / 4.3, Q2_K 5.1 / 4.4).
-    p.waves = nsub <= 16 ? 4 : nsub < 64 ? 8 : 16;
+    // Where each workgroup has a CU to itself 16 waves from 32 sub-blocks on, 40 for
+    // the formats that decode in fewer steps (1024 x 1024 at 8 rows, 8 / 16 waves:
+    // Q4_K 4.8 / 4.5, Q8_0 3.8 / 3.8; 1280 x 300 Q6_K 5.9 / 5.4, Q4_1 5.5 / 5.2).
+    const int most8 = blocks > kCus ? 64 : fmt <= kQ5_1 ? 40 : 32;
+    p.waves = nsub <= 16 ? 4 : nsub < most8 ? 8 : 16;
     const int per = (nsub + p.waves - 1) / p.waves, runs = (per + 3) / 4;
     p.depth = (per + runs - 1) / runs;
     if (p.depth < 2) p.depth = 2;
