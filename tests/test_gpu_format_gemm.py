@@ -4,9 +4,12 @@ sub-blocks. Reference: the session's own dequantized weights (bit-identical
 to the oracle's, test_gpu_formats.py) times x in f64. Bound: exact codes and
 x to 2^-25, fp32 sums over K/32 sub-blocks of a wave: a few 2^-24, 2e-6 with the
 cancellation of N(0, 1) inputs."""
+import ctypes
+
 import numpy as np
 import pytest
 
+import launch_rules
 from test_gpu_dense import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -116,3 +119,31 @@ def test_format_gemm_non_finite_inputs(gpu, fmt):
 ])
 def test_format_small_products_match_f64(gpu, fmt, batch, inp, out):
     test_format_gemm_matches_f64(gpu, fmt, batch, inp, out)
+
+
+@pytest.mark.parametrize("batch,kernel,copies", [(1, launch_rules.PER_ROW, 1), (4, launch_rules.PER_ROW, 1),
+                                                 (8, launch_rules.ROWS, 2)])
+def test_second_copy_of_the_weights_only_where_it_is_read(gpu, batch, kernel, copies):
+    """Device memory of four mounted Q4_0 layers of 59 MB of blocks each: twice
+    that for a batch of the matrix-core kernels, which read an interleaved copy.
+    (The runtime may keep one more freed buffer of that size.)"""
+    inp, out, fmt, layers = 32768, 3200, 2, 4
+    assert launch_rules.format_plan(fmt, out, inp, batch).kernel == kernel
+    h = gpu.Hip()
+
+    def used():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        h.sync()
+        assert h.h.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return total.value - free.value
+
+    nbytes = inp * out // 32 * 18
+    blocks = np.zeros(nbytes, np.uint8)
+    mount = lambda: gpu.FormatDenseSession(batch, inp, out, gpu.LINEAR, fmt, blocks=blocks)
+    mount().close()  # what the library allocates once
+    before = used()
+    sessions = [mount() for _ in range(layers)]
+    held = used() - before
+    for s in sessions:
+        s.close()
+    assert abs(held / layers - copies * nbytes) < 0.5 * nbytes

@@ -295,8 +295,10 @@ static Status build_frag(DenseLayer* L, hipStream_t st) {
 
 Status dense_prepare_rows(DenseLayer* L, int batch, hipStream_t st) {
   if (L->format) {
+    // a second copy only for a batch whose kernel reads it
     FormatWeights& f = L->fw;
-    if (batch < format_rows_batch(f.format) || f.il.p) return Status::ok();
+    if (f.il.p || format_plan(f.format, f.rows, f.nsub, batch).kernel == FmtKernel::kPerRow)
+      return Status::ok();
     WV_TRY(f.il.alloc(format_interleaved_bytes(f.format, f.rows, f.nsub)));
     WV_TRY(format_interleave(f.format, format_args(*L), f.il.as<uint8_t>(), f.rpad, &f.tiles, st));
     return hip_status(hipStreamSynchronize(st), "format interleave");
