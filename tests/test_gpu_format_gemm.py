@@ -5,11 +5,13 @@ to the oracle's, test_gpu_formats.py) times x in f64. Bound: exact codes and
 x to 2^-25, fp32 sums over K/32 sub-blocks of a wave: a few 2^-24, 2e-6 with the
 cancellation of N(0, 1) inputs."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
 
 import launch_rules
+from format_blocks import random_blocks
 from test_gpu_dense import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -119,6 +121,36 @@ def test_format_gemm_non_finite_inputs(gpu, fmt):
 ])
 def test_format_small_products_match_f64(gpu, fmt, batch, inp, out):
     test_format_gemm_matches_f64(gpu, fmt, batch, inp, out)
+
+
+@pytest.mark.parametrize("fmt", [1, 10])
+def test_all_nan_batch_costs_no_recompute(gpu, fmt):
+    """A diverged batch, NaN all over, is recomputed to the first NaN of each output
+    only: within a few times the clean batch's time (33 times with whole rows)."""
+    h = gpu.Hip()
+    batch, n = 512, 2048
+    s = gpu.FormatDenseSession(batch, n, n, gpu.LINEAR, fmt,
+                               blocks=random_blocks(fmt, n, n, np.random.default_rng(fmt)))
+    clean = h.upload(np.ones((batch, n), np.float32))
+    nan = h.upload(np.full((batch, n), np.nan, np.float32))
+    y = h.malloc(batch * n * 4)
+
+    def seconds(x):
+        best = 1e9
+        for _ in range(20):
+            h.sync()
+            t = time.perf_counter()
+            s.execute_device(x, y, y)
+            h.sync()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    a, b = seconds(clean), seconds(nan)
+    assert np.isnan(h.download(y, (batch, n))).all()
+    s.close()
+    for p in (clean, nan, y):
+        h.free(p)
+    assert b <= 4 * a
 
 
 @pytest.mark.parametrize("batch,kernel,copies", [(1, launch_rules.PER_ROW, 1), (4, launch_rules.PER_ROW, 1),

@@ -1225,11 +1225,14 @@ __device__ __forceinline__ void fmt_scales(const FmtRaw& r, int t, float (&d)[2]
 }
 
 // One output over the dequantized weights, for a sum that is not finite: the
-// bf16 terms of an infinity (or of a value that rounds to one) are NaN.
+// bf16 terms of an infinity (or of a value that rounds to one) are NaN. It ends at
+// the first NaN, so that a diverged batch, NaN all over, costs what a clean one
+// does (512 rows of 4096 x 4096 Q8_0: 2247 us without that end, 81 with it, 68
+// clean); an infinity in every row still takes 2247.
 template <int FMT>
 __device__ float fmt_dot(const FmtArgs& a, int row, const float* __restrict__ x) {
   float v = 0.0f;
-  for (int t = 0; t < a.nsub; ++t) {
+  for (int t = 0; t < a.nsub && v == v; ++t) {
     float w[32];
     dequant_sub<FMT>(a, row, t, w);
 #pragma unroll
