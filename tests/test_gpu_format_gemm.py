@@ -1,6 +1,8 @@
-"""The block formats' matrix-core product at the edges of its tiles: 32 or 64
-batch rows by 32, 64 or 128 weight rows, K split over 4 or 8 waves in 32-element
-sub-blocks. Reference: the session's own dequantized weights (bit-identical
+"""The block formats' matrix-core products at the edges of their tiles: 16
+batch rows by 16 weight rows with K split over 4, 8 or 16 waves, and 32 or 64 batch
+rows by 32, 64 or 128 weight rows with K split over 8, in 32-element sub-blocks.
+Tests that are meant for one of them ask the launch rule that it takes their sizes.
+Reference: the session's own dequantized weights (bit-identical
 to the oracle's, test_gpu_formats.py) times x in f64. Bound: exact codes and
 x to 2^-25, fp32 sums over K/32 sub-blocks of a wave: a few 2^-24, 2e-6 with the
 cancellation of N(0, 1) inputs."""
@@ -30,16 +32,20 @@ def weights(rng, out, inp):
 @pytest.mark.parametrize("batch,inp,out", [
     (8, 256, 33),      # the least batch; one weight row past a tile
     (31, 768, 64),     # 24 sub-blocks over 8 waves
-    (32, 1280, 16),    # fewer weight rows than a tile
-    (33, 512, 97),     # two 32-row blocks, ragged weight tile
-    (97, 256, 200),    # last 64-row tile half empty
+    (32, 1280, 16),    # as many weight rows as a tile
+    (33, 512, 97),     # three 16-row blocks, ragged weight tile
+    (97, 256, 200),    # last 16-row block nearly empty
     (385, 256, 1800),  # 64 x 64 tiles, ragged on both sides
-    (200, 512, 6100),  # 64 x 128 tiles, 4 waves
+    (200, 512, 6100),  # 64 x 128 tiles
 ])
 def test_format_gemm_matches_f64(gpu, fmt, batch, inp, out):
-    rng = np.random.default_rng(fmt * 1000 + batch + out)
     if fmt not in SUPER:
         inp += 96  # a number of sub-blocks that no wave count divides
+    check_against_f64(gpu, fmt, batch, inp, out)
+
+
+def check_against_f64(gpu, fmt, batch, inp, out):
+    rng = np.random.default_rng(fmt * 1000 + batch + out)
     s = gpu.FormatDenseSession(batch, inp, out, gpu.LINEAR, fmt, W=weights(rng, out, inp))
     x = rng.standard_normal((batch, inp)).astype(np.float32)
     x *= np.exp(rng.uniform(-6, 6, (batch, 1))).astype(np.float32)
@@ -53,12 +59,49 @@ def test_format_gemm_matches_f64(gpu, fmt, batch, inp, out):
     assert rel_l2(y, want) <= 2e-6
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("batch,inp,out,tile", [
+    (33, 3072, 2081, (1, 1)),   # two 32-row blocks, the second with one row
+    (40, 2560, 1376, (1, 1)),
+    (128, 512, 4096, (1, 2)),   # exact tiles
+    (97, 512, 5601, (1, 2)),    # one row past the last block on both sides
+    (385, 512, 1800, (2, 2)),
+    (200, 512, 6100, (2, 4)),
+])
+def test_each_gemm_tile_matches_f64(gpu, fmt, batch, inp, out, tile):
+    for i in (inp, inp + 96):
+        p = launch_rules.format_plan(fmt, out, i, batch)
+        assert (p.kernel, p.tm, p.tn) == (launch_rules.GEMM,) + tile
+    test_format_gemm_matches_f64(gpu, fmt, batch, inp, out)
+
+
+@pytest.mark.parametrize("fmt,batch,inp,out,shape", [
+    (2, 9, 64, 33, (4, 2)), (8, 16, 256, 33, (4, 2)),
+    (2, 17, 352, 40, (4, 3)), (5, 8, 288, 40, (4, 3)),  # (11 and 9 sub-blocks: 3 and 2 a wave)
+    (3, 9, 512, 20, (4, 4)), (9, 16, 512, 20, (4, 4)),
+    (1, 8, 768, 33, (8, 3)), (6, 20, 768, 33, (8, 3)), (7, 8, 768, 33, (8, 3)),
+    (4, 16, 1024, 17, (8, 4)), (10, 16, 1024, 4161, (8, 4)), (6, 16, 1024, 4161, (8, 4)),
+    (8, 16, 1024, 513, (16, 2)), (6, 8, 1024, 513, (16, 2)), (7, 40, 1024, 100, (16, 2)),
+    (2, 16, 1280, 33, (16, 3)), (10, 12, 1536, 33, (16, 3)), (3, 16, 4672, 20, (16, 4)),
+    (17, 16, 2048, 50, (16, 4)), (6, 16, 4096, 50, (16, 4)),
+])
+def test_each_small_product_shape_matches_f64(gpu, fmt, batch, inp, out, shape):
+    """Every built (waves, sub-blocks ahead) of the 16 x 16 blocks."""
+    p = launch_rules.format_plan(fmt, out, inp, batch)
+    assert (p.kernel, p.waves, p.depth) == (launch_rules.ROWS,) + shape
+    check_against_f64(gpu, fmt, batch, inp, out)
+
+
 @pytest.mark.parametrize("fmt", [1, 8])
-def test_format_gemm_epilogue_and_row_runs(gpu, fmt):
+@pytest.mark.parametrize("out,kernel", [(40, launch_rules.ROWS), (80, launch_rules.GEMM)])
+def test_format_gemm_epilogue_and_row_runs(gpu, fmt, out, kernel):
     """Bias and activation, and rows that the scratch holds in several runs
     (the allocation-free execute has 64 MiB): the same bits as one run."""
     rng = np.random.default_rng(fmt)
-    batch, inp, out = 1000, 16384, 40
+    batch, inp = 1000, 16384
+    plan = launch_rules.format_plan(fmt, out, inp, batch)
+    assert plan.kernel == kernel
+    assert kernel == launch_rules.ROWS or plan.run_rows < batch
     bias = rng.standard_normal(out)
     s = gpu.FormatDenseSession(batch, inp, out, gpu.SILU, fmt, W=weights(rng, out, inp), bias=bias)
     x = rng.standard_normal((batch, inp)).astype(np.float32)
@@ -79,12 +122,14 @@ def test_format_gemm_epilogue_and_row_runs(gpu, fmt):
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
-def test_format_gemm_non_finite_inputs(gpu, fmt):
+@pytest.mark.parametrize("out,kernel", [(70, launch_rules.ROWS), (5600, launch_rules.GEMM)])
+def test_format_gemm_non_finite_inputs(gpu, fmt, out, kernel):
     """A row of x with an infinity, a NaN or values near the f32 maximum (whose
     bf16 terms overflow) gives the dequantized product's result there and
     leaves the other rows alone."""
     rng = np.random.default_rng(fmt + 50)
-    batch, inp, out = 40, 512, 70
+    batch, inp = 40, 512
+    assert launch_rules.format_plan(fmt, out, inp, batch).kernel == kernel
     s = gpu.FormatDenseSession(batch, inp, out, gpu.LINEAR, fmt, W=weights(rng, out, inp))
     x = rng.standard_normal((batch, inp)).astype(np.float32)
     clean, _ = s.execute(x)
@@ -117,7 +162,7 @@ def test_format_gemm_non_finite_inputs(gpu, fmt):
     (100, 768, 160),  # 7 batch blocks, the last with 4 rows
     (33, 2048, 400),  # 16 waves, 3 batch blocks
     (40, 2048, 1360),  # 85 x 3 blocks, the last count below 256
-    (40, 2048, 1376),  # 86 x 3: the split and the larger tiles
+    (40, 2048, 1376),  # 86 x 3
 ])
 def test_format_small_products_match_f64(gpu, fmt, batch, inp, out):
     test_format_gemm_matches_f64(gpu, fmt, batch, inp, out)

@@ -125,7 +125,7 @@ def test_mount_from_blocks_dequant_and_export(gpu, oracle, fmt, rows, cols):
 @pytest.mark.parametrize("fmt", ALL, ids=lambda f: NAMES[f])
 @pytest.mark.parametrize("batch", [1, 3, 8, 16, 37])
 def test_gemv_against_oracle(gpu, oracle, fmt, batch):
-    """Batches below 8 run the per-row kernel, from 8 the matrix-core one
+    """Batches of 1 and 3 run the per-row kernel, from 8 the matrix-core one
     (37: three groups of 16 batch rows, the last ragged)."""
     rng = np.random.default_rng(fmt * 31 + batch)
     rows, cols = 333, 2048
