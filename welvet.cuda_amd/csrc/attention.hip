@@ -14,6 +14,7 @@
 // the softmax is accumulated online in fp32. RoPE is applied by the Q and K
 // projections' GEMM epilogue when they run on the large tiles, else by
 // k_rope before either kernel.
+#include "bf16.h"
 #include "common.h"
 #include "kernels.h"
 #include "split.h"
@@ -276,7 +277,7 @@ __device__ __forceinline__ int key_count(const AttnArgs& a, int p, int qp, int l
 // e^(-s msl) near 1, keeps too few digits at the flattest slope (2^-8): 4e-6 of a
 // weight at 2 rows, from 16 on below the exponents' own rounding. SHORT takes
 // r^c - 1 over r - 1 from expm1f instead, in kernels of its own (expm1f in the
-// others costs them up to 7%, in registers also where it is not run).
+// others costs them up to 5%, also where it is not run).
 constexpr int kShortRing = 16;
 
 // The ALiBi constants of a head: the slope in log2 units and, for the sums
@@ -308,19 +309,6 @@ __device__ __forceinline__ float log2_weight(const AttnArgs& a, int p, int qp, i
   const float up = -s.sl2 * (float)(p - qp);
   const float m = fmaxf(up, below);
   return m + __builtin_amdgcn_logf(__builtin_amdgcn_exp2f(up - m) + __builtin_amdgcn_exp2f(below - m));
-}
-
-// x as T bf16 terms, each rounding the remainder of the ones before it (to
-// nearest even): two leave 2^-17 |x|, three 2^-25 |x|.
-template <int T>
-__device__ __forceinline__ void split_bf16(v4f x, bf16x4 (&t)[T]) {
-#pragma unroll
-  for (int k = 0; k < T; ++k)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      t[k][e] = (__bf16)x[e];
-      x[e] -= (float)t[k][e];
-    }
 }
 
 // acc + A B with both operands in T bf16 terms: the products a_i b_j with

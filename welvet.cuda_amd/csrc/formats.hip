@@ -28,6 +28,7 @@
 // padded to a multiple of 16 with zero bytes (zero scales: padding rows read
 // as 0).
 #include "act.h"
+#include "bf16.h"
 #include "common.h"
 #include "kernels.h"
 #include "wave.h"
@@ -976,6 +977,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_fmt_gemv(FmtArgs a) {
 // reaches 1290). The products bound it: with a third of them it takes 46 us;
 // without the loads of x 60, of the weights 63.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float v8f __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr bool fmt_halves(int fmt) { return fmt == kQ6_K; }
@@ -983,15 +985,6 @@ constexpr bool fmt_scaled_codes(int fmt) { return fmt == kQ2_K || fmt == kQ3_K; 
 // bytes of the super-block header that holds the scales, if the format has one
 constexpr int fmt_header(int fmt) {
   return fmt == kQ4_K || fmt == kQ5_K || fmt == kQ3_K ? 16 : fmt == kIQ4_XS ? 8 : 0;
-}
-
-// v as three bf16 terms, each rounding the remainder of those before it.
-__device__ __forceinline__ void fmt_terms(float v, __bf16 (&t)[3]) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    t[k] = (__bf16)v;
-    v -= (float)t[k];
-  }
 }
 
 // One workgroup per 32 batch rows x 128 columns, staged in LDS with
@@ -1025,25 +1018,19 @@ __global__ __launch_bounds__(kThreads) void k_fmt_split(const float* __restrict_
   for (int s = 0; s < 2; ++s) {
     const v4f lo = *reinterpret_cast<const v4f*>(src + 16 * s);
     const v4f hi = *reinterpret_cast<const v4f*>(src + 16 * s + 4);
-    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    const v8f v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     sum[s] = 0.0f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) sum[s] += v[j];
+    bf16x8 c[3];
+    split_bf16<3>(v, c);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      bf16x8 c;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        c[j] = (__bf16)v[j];
-        v[j] -= (float)c[j];
-      }
-      *reinterpret_cast<bf16x8*>(dst + (2 * k + s) * 1024) = c;
-    }
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + (2 * k + s) * 1024) = c[k];
     if constexpr (AFFINE) sum[s] += __shfl_xor(sum[s], 32, 64);
   }
   if constexpr (AFFINE) {
     __bf16 u[3];
-    fmt_terms(half == 0 ? sum[0] : sum[1], u);
+    split_bf16<3>(half == 0 ? sum[0] : sum[1], u);
     const __bf16 z = (__bf16)0.0f;
     const bf16x8 c = {u[0], u[0], u[1], u[0], u[1], u[2], z, z};
     *reinterpret_cast<bf16x8*>(dst + 6 * 1024) = c;
@@ -1335,7 +1322,7 @@ __global__ __launch_bounds__(64 * W) void k_fmt_gemm(FmtArgs a, FmtArgs plain,
       bf16x8 bo;
       if constexpr (AFFINE) {
         __bf16 u[3];
-        fmt_terms(half == 0 ? off[0] : off[1], u);
+        split_bf16<3>(half == 0 ? off[0] : off[1], u);
         const __bf16 z = (__bf16)0.0f;
         bo = bf16x8{u[0], u[1], u[0], u[2], u[1], u[0], z, z};
       }
@@ -1456,12 +1443,11 @@ __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, i
       bf16x8 bo = zero;
       if constexpr (AFFINE) {
         __bf16 c[3];
-        fmt_terms(g < 2 ? off[0] : off[1], c);
+        split_bf16<3>(g < 2 ? off[0] : off[1], c);
         if ((g & 1) == 0) bo = bf16x8{c[0], c[1], c[0], c[2], c[1], c[0], zero[0], zero[0]};
       }
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = xv[u][j >> 2][j & 3];
+      const v4f lo = xv[u][0], hi = xv[u][1];
+      const v8f v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       float sum = 0.0f;
       if constexpr (AFFINE) {
 #pragma unroll
@@ -1469,13 +1455,7 @@ __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, i
         sum += __shfl_xor(sum, 16, 64);
       }
       bf16x8 x[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          x[k][j] = (__bf16)v[j];
-          v[j] -= (float)x[k][j];
-        }
+      split_bf16<3>(v, x);
       v4f d0 = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 2; k >= 0; --k) d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[k], b0, d0, 0, 0, 0);
@@ -1490,7 +1470,7 @@ __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, i
       }
       if constexpr (AFFINE) {
         __bf16 c[3];
-        fmt_terms(sum, c);
+        split_bf16<3>(sum, c);
         const bf16x8 xo = {c[0], c[0], c[1], c[0], c[1], c[2], zero[0], zero[0]};
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xo, bo, acc, 0, 0, 0);
       }
