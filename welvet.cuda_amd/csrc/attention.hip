@@ -227,7 +227,7 @@ __global__ __launch_bounds__(64) void k_attention(AttnArgs a) {
 // the output is 1e-7 off, as the fp32 loop of k_attention that it replaces.
 // That loop took one wave per (token, head) and one dependent V row per key:
 // 3 x 701 tokens, 12 heads of 64 over 4 K/V heads, causal with ALiBi: the layer
-// 1636 us, now 134 us (this kernel about 75 us; its matrix-core work is 20 us,
+// 1636 us, now 109 us (this kernel 71 us; its matrix-core work is 14 us,
 // the softmax, the splits and the LDS traffic of two waves per SIMD the rest).
 // Keys per LDS tile: 64; 32 for GEN at 128 head dims (three terms of 64 keys
 // do not fit the LDS twice) and for the 4-wave workgroups whose 64 keys would

@@ -972,7 +972,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_fmt_gemv(FmtArgs a) {
 // wave of the SIMD. The weights are read from an interleaved copy, whose loads
 // are contiguous (row-major, a load touches 32 rows' lines: 80 instead of 62 us).
 // 4096 x 4096, 512 rows, Q8_0: 455 us on fp32 matrix products that decoded every
-// weight once per 16 batch rows, now 62 us with the split; 512 more rows take
+// weight once per 16 batch rows, now 59 us with the split; 512 more rows take
 // 53 us (970 TFLOP/s of bf16 products, where a plain bf16 product of torch
 // reaches 1290). The products bound it: with a third of them it takes 46 us;
 // without the loads of x 60, of the weights 63.
@@ -1401,7 +1401,7 @@ __global__ __launch_bounds__(64 * W) void k_fmt_gemm(FmtArgs a, FmtArgs plain,
 // two with the other half zeroed for fmt_halves). Bound by the latency of its
 // loads: those of `kDepth` sub-blocks are issued before the first of them is
 // used, and 16 waves make it two rounds at 4096 columns. 4096 x 4096 Q4_0 at 8
-// rows 10.2 us (13.0 on the fp32 matrix products), at 4 rows 9.6 us (11.6 with
+// rows 8.8 us (13.0 on the fp32 matrix products), at 4 rows 8.4 us (11.6 with
 // every batch row streaming the weights); from row-major weights 14.9. Fewer
 // sub-blocks feed fewer waves (format_plan).
 template <int FMT, int W, int kDepth>
