@@ -168,6 +168,31 @@ def test_format_small_products_match_f64(gpu, fmt, batch, inp, out):
     test_format_gemm_matches_f64(gpu, fmt, batch, inp, out)
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("batch,out,kernel", [(16, 70, launch_rules.ROWS), (40, 5600, launch_rules.GEMM)])
+def test_format_gemm_small_inputs(gpu, fmt, batch, out, kernel):
+    """Inputs down to f32's least normals keep fp32's digits, beside rows of
+    ordinary size, and zeros stay zeros: bf16 terms of a value end at 2^-133.
+    Bound: the products' 2e-6, and from 2^-120 on the rounding of outputs near the
+    least normal (2^-149 of 2^-126 and less)."""
+    rng = np.random.default_rng(fmt)
+    inp = 512
+    assert launch_rules.format_plan(fmt, out, inp, batch).kernel == kernel
+    s = gpu.FormatDenseSession(batch, inp, out, gpu.LINEAR, fmt, W=weights(rng, out, inp))
+    x = rng.standard_normal((batch, inp)).astype(np.float32)
+    x[1:6] *= np.float32(2) ** -np.array([[60], [96], [104], [112], [118]], np.float32)
+    x[6] = 0.0
+    y, _ = s.execute(x)
+    W = s.export_f32().astype(np.float64)
+    s.close()
+    want = x.astype(np.float64) @ W.T
+    assert not y[6].any()
+    for r in range(batch):
+        if r != 6:
+            k = 2.0 ** 126 if 1 <= r < 6 else 1.0
+            assert rel_l2(y[r] * k, want[r] * k) <= 2e-6
+
+
 @pytest.mark.parametrize("fmt", [1, 10])
 def test_all_nan_batch_costs_no_recompute(gpu, fmt):
     """A diverged batch, NaN all over, is recomputed to the first NaN of each output

@@ -1211,8 +1211,11 @@ __device__ __forceinline__ void fmt_scales(const FmtRaw& r, int t, float (&d)[2]
   }
 }
 
-// One output over the dequantized weights, for a sum that is not finite: the
-// bf16 terms of an infinity (or of a value that rounds to one) are NaN. It ends at
+// One output over the dequantized weights, in fp32 from the first element to the
+// last: for a sum that is not finite (the bf16 terms of an infinity, or of a value
+// that rounds to one, are NaN), and for one so small that x must be below 2^-100 or
+// so, where its third term, and then its second, falls under bf16's least
+// subnormal, 2^-133 (x near 2^-120: 3.5e-5 relative, near 2^-128 9e-3). It ends at
 // the first NaN, so that a diverged batch, NaN all over, costs what a clean one
 // does (512 rows of 4096 x 4096 Q8_0: 2247 us without that end, 81 with it, 68
 // clean); an infinity in every row still takes 2247.
@@ -1245,7 +1248,11 @@ __device__ __forceinline__ float add_waves(F sum) {
 // The Dense epilogue of output (batch row j, weight row o).
 template <int FMT>
 __device__ __forceinline__ void fmt_store(const FmtArgs& a, int j, int o, float v) {
-  if (!(v - v == 0.0f)) v = fmt_dot<FMT>(a, o, a.x + (size_t)j * a.x_stride);
+  // outside [2^-90, infinity) (what x's terms lose is at most 2^-134 of each
+  // weight: nothing to a sum of 2^-90); zeros stay
+  const uint32_t size = __float_as_uint(v) & 0x7FFFFFFFu;
+  if (size - 0x12800000u >= 0x7F800000u - 0x12800000u && size != 0)
+    v = fmt_dot<FMT>(a, o, a.x + (size_t)j * a.x_stride);
   const size_t oi = (size_t)j * a.out_stride + o;
   if (a.need_epi) {
     double d = (double)v;
