@@ -1091,6 +1091,19 @@ __device__ __forceinline__ void fmt_load(const FmtArgs& a, const FmtRow& row, in
   if constexpr (G.eb == 4) r.e = *reinterpret_cast<const uint32_t*>(a.e + super * 4);
 }
 
+// The loaded values are in registers from here on: a branch that follows, over
+// their only use, does not take their loads along.
+template <int FMT>
+__device__ __forceinline__ void fmt_loaded(FmtRaw& r, v4f (&x)[2]) {
+  constexpr FmtGeom G = fmt_geom(FMT);
+  asm volatile("" : "+v"(r.w[0]), "+v"(r.w[1]), "+v"(r.s[0]), "+v"(x[0]), "+v"(x[1]));
+  if constexpr (G.hb >= 4) asm volatile("" : "+v"(r.h0));
+  if constexpr (G.hb == 8) asm volatile("" : "+v"(r.h1));
+  if constexpr (fmt_header(FMT) >= 8) asm volatile("" : "+v"(r.s[1]));
+  if constexpr (fmt_header(FMT) == 16) asm volatile("" : "+v"(r.s[2]), "+v"(r.s[3]));
+  if constexpr (G.eb > 0) asm volatile("" : "+v"(r.e));
+}
+
 // The interleaved copy of one array: records of `bytes` (2, 4, 8, 16 or 32),
 // n per row, from [row][n] to [row / 32][n][row % 32]; rows past the source
 // are zeros. One thread per 2 bytes, the destination's neighbours in turn.
@@ -1410,7 +1423,11 @@ __global__ __launch_bounds__(64 * W) void k_fmt_gemm(FmtArgs a, FmtArgs plain,
 // used, and 16 waves make it two rounds at 4096 columns. 4096 x 4096 Q4_0 at 8
 // rows 8.8 us (13.0 on the fp32 matrix products), at 4 rows 8.4 us (11.6 with
 // every batch row streaming the weights); from row-major weights 14.9. Fewer
-// sub-blocks feed fewer waves (format_plan).
+// sub-blocks feed fewer waves (format_plan). The VALU bounds it where a workgroup
+// walks many sub-blocks (about 100 to 150 operations each, most of them the split of
+// x): a run's sub-blocks past the wave's last one are skipped, and the waves that
+// have one more are spread over the SIMDs (2304 x 300 at 8 rows, 4.5 sub-blocks a
+// wave: Q6_K 8.5 -> 7.4 us, Q2_K 8.9 -> 7.5).
 template <int FMT, int W, int kDepth>
 __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, int batch) {
   constexpr bool HALVES = fmt_halves(FMT), AFFINE = fmt_affine(FMT);
@@ -1418,7 +1435,10 @@ __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, i
   const int i16 = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
   const FmtRow row = fmt_row(a, n0 + i16 < a.rows ? n0 + i16 : a.rows - 1);
-  const int t0 = (int)((int64_t)a.nsub * wave / W), t1 = (int)((int64_t)a.nsub * (wave + 1) / W);
+  // (the first waves take one more: every fourth wave shares a SIMD, which
+  // spreads them evenly)
+  const int base = a.nsub / W, extra = a.nsub % W;
+  const int t0 = wave * base + (wave < extra ? wave : extra), t1 = t0 + base + (wave < extra ? 1 : 0);
   // (lanes past the last batch row read row 0: a product's rows stay apart, and
   // theirs are not stored)
   const float* src = a.x + (size_t)(m0 + i16 < batch ? m0 + i16 : 0) * a.x_stride + 8 * g;
@@ -1438,12 +1458,10 @@ __global__ __launch_bounds__(64 * W) void k_fmt_rows(FmtArgs a, FmtArgs plain, i
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kDepth; ++u) {
+      fmt_loaded<FMT>(raw[u], xv[u]);
+      if (tb + u >= t1) break;  // wave-uniform
       float d[2], off[2], mul[2];
-      fmt_scales<FMT>(raw[u], tb + u < t1 ? tb + u : t1 - 1, d, off, mul);
-      // past the range: the last sub-block again, times 0 (a branch here would
-      // take the loads along)
-      const float on = tb + u < t1 ? 1.0f : 0.0f;
-      d[0] *= on, d[1] *= on, off[0] *= on, off[1] *= on;
+      fmt_scales<FMT>(raw[u], tb + u, d, off, mul);
       const bf16x8 b = fmt_codes8<FMT>({raw[u].w[0], raw[u].w[1]}, raw[u].h0, raw[u].h1, g,
                                           g < 2 ? mul[0] : mul[1]);
       const bf16x8 b0 = HALVES && g >= 2 ? zero : b, b1 = g < 2 ? zero : b;

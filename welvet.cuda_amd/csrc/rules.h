@@ -100,7 +100,7 @@ inline FmtPlan format_plan(int fmt, int rows, int nsub, int batch) {
     // 512 x 256 4.1 / 4.1 / 5.4 (Q4_K 3.9 / 4.7 / 6.6), 1024 x 1024 4.5 / 4.1 /
     // 5.5, 768 x 6400 6.0 / 5.7 / 9.2, 2048 x 2048 6.8 / 5.8 / 5.6, 2048 x 4096 6.8 /
     // 5.9 / 5.7. A wave loads all of its sub-blocks ahead, or equal runs of at most
-    // 4: what a run holds past the last one is work for nothing (256 x 8192 at 16
+    // 4: what a run holds past the last one is loaded for nothing (256 x 8192 at 16
     // rows, 2 sub-blocks a wave, with runs of 4 / 2: Q4_0 4.6 / 3.6, Q6_K 5.2 / 3.8;
     // 768 x 448, 3 a wave, with 4 / 3: Q6_K 4.9 / 4.3, Q2_K 5.1 / 4.4).
     // Where each workgroup has a CU to itself 16 waves from 32 sub-blocks on, 40 for
